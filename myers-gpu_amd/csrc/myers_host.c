@@ -43,6 +43,7 @@
 #define STAGE_BYTES      (64u << 20)    /* pinned staging for the reference upload */
 #define DEFAULT_BUFFER_CAP (2ull << 30)
 #define EV_RING          32u            /* kernel-timing event pairs per buffer */
+#define GROUP_N_WORDS    12u             /* reads of more words: candidates grouped by N in the read */
 #define SIDE_STREAMS     4u             /* fork width of a persistent launch */
 
 typedef struct myers_ctx {
@@ -52,19 +53,21 @@ typedef struct myers_ctx {
     uint64_t  ref_words;         /* stored words */
     uint64_t  ref_words_alloc;   /* stored + guard */
     uint64_t  ref_size;          /* bases */
+    uint32_t *d_planes;          /* bit planes of d_ref for the one-lane variants */
+    uint32_t  plane_blocks;
     uint32_t  num_variants;
     myers_variant_desc_t variants[MYERS_MAX_VARIANTS];
     int       occupancy[MYERS_MAX_VARIANTS];       /* plain kernel, workgroups per CU */
     int       occupancy_p[MYERS_MAX_VARIANTS];     /* persistent kernel */
     uint32_t  chunk_factor[MYERS_MAX_VARIANTS];    /* persistent: chunks per queue pull */
     uint32_t  long_seq;                            /* long-read launches so far (placement rotation) */
-    int       queue_occ[MYERS_QUEUE_CLASSES][2];   /* queue kernel workgroups per CU, [class][cut], */
-    uint32_t  queue_occ_lds[MYERS_QUEUE_CLASSES][2];  /* for this dynamic LDS size (0: not queried) */
+    int       queue_occ[4];                        /* workgroups per CU of the multi-lane queue kernel, its
+                                                      threshold form and the two one-lane kernels, */
+    uint32_t  queue_occ_lds[4];                    /* for this dynamic LDS size (0: not queried) */
     uint8_t   bin_of_words[MAX_QUERY_WORDS + 1];
     uint8_t  *d_bin_of_words;
     uint64_t  tune_gen;          /* bumped when the bin table or chunk factors change */
     uint32_t *d_scratch;         /* this device's static workspace (myersVerifyDeviceNoAlloc) */
-    uint64_t  probe_mask;        /* threshold mode: variants whose candidates the band probe orders */
 } myers_ctx_t;
 
 typedef struct myers_buffer {
@@ -252,8 +255,10 @@ static int upload_reference(myers_ctx_t *ctx, const uint32_t *words, uint64_t nu
     size_t free_b = 0, total_b = 0;
     HIP_TRY(hipMemGetInfo(&free_b, &total_b));
     const uint64_t bytes = (num_words + GUARD_WORDS) * sizeof(uint32_t);
-    if (bytes > free_b) return MYERS_E_INSUFFICIENT_MEM_GPU;
+    const uint64_t blocks = (num_words + GUARD_WORDS + 3u) / 4u;        /* 32 bases each */
+    if (bytes + 3u * sizeof(uint32_t) * blocks > free_b) return MYERS_E_INSUFFICIENT_MEM_GPU;
     HIP_TRY(hipMalloc((void **)&ctx->d_ref, bytes));
+    HIP_TRY(hipMalloc((void **)&ctx->d_planes, 3u * sizeof(uint32_t) * blocks));
     /* Stream the words through a pinned staging buffer. */
     void *stage = NULL;
     size_t stage_bytes = STAGE_BYTES;
@@ -272,7 +277,10 @@ static int upload_reference(myers_ctx_t *ctx, const uint32_t *words, uint64_t nu
     hipHostFree(stage);
     if (rc) return rc;
     HIP_TRY(hipMemsetD32((hipDeviceptr_t)(ctx->d_ref + num_words), (int)ALL_N_WORD, GUARD_WORDS));
+    rc = myers_launch_planes(ctx->d_ref, num_words + GUARD_WORDS, ctx->d_planes, (uint32_t)blocks, NULL);
+    if (rc) return hip_fail((hipError_t)rc, "reference planes launch", __FILE__, __LINE__);
     HIP_TRY(hipDeviceSynchronize());
+    ctx->plane_blocks = (uint32_t)blocks;
     ctx->ref_words = num_words;
     ctx->ref_words_alloc = num_words + GUARD_WORDS;
     ctx->ref_size = size;
@@ -364,7 +372,6 @@ static int create_context(myers_ctx_t **out, int device)
         return MYERS_E_HIP;
     }
     ctx->num_variants = myers_num_variants();
-    ctx->probe_mask = myers_probe_variants();
     for (uint32_t v = 0; v < ctx->num_variants; v++) {
         myers_variant_desc(v, &ctx->variants[v]);
         int occ = 0;
@@ -395,6 +402,7 @@ static void free_context(myers_ctx_t *ctx)
 {
     if (ctx == NULL) return;
     if (ctx->d_ref) hipFree(ctx->d_ref);
+    if (ctx->d_planes) hipFree(ctx->d_planes);
     if (ctx->d_bin_of_words) hipFree(ctx->d_bin_of_words);
     free(ctx);
 }
@@ -750,38 +758,136 @@ static uint32_t long_plan(const myers_ctx_t *ctx, const bin_scan_t *scan, const 
     return nt;
 }
 
-/* Resident workgroups per CU of a queue kernel with `lds` bytes of
- * dynamic LDS (queried once per size). */
-static uint32_t queue_grid(myers_ctx_t *ctx, uint32_t cls, int cut, uint32_t lds)
+/* Workgroups of a resident grid of the multi-lane queue kernel (which = 0, 1:
+ * its threshold form) or a one-lane kernel (2: 16 lanes per group, 3: 32) with
+ * `lds` bytes of dynamic LDS (queried once per size). */
+static uint32_t queue_grid(myers_ctx_t *ctx, uint32_t which, uint32_t lds)
 {
-    if (ctx->queue_occ_lds[cls][cut] != lds) {
+    if (ctx->queue_occ_lds[which] != lds) {
         int occ = 0;
-        if (myers_queue_occupancy(cls, cut, lds, &occ) != 0 || occ <= 0) occ = 1;
-        ctx->queue_occ[cls][cut] = occ;
-        ctx->queue_occ_lds[cls][cut] = lds;
+        const int rc = which >= 2u ? myers_slice_occupancy(16u * (which - 1u), lds, &occ) : myers_queue_occupancy((int)which, lds, &occ);
+        if (rc != 0 || occ <= 0) occ = 1;
+        ctx->queue_occ[which] = occ;
+        ctx->queue_occ_lds[which] = lds;
     }
-    return (uint32_t)ctx->num_cus * (uint32_t)ctx->queue_occ[cls][cut];
+    return (uint32_t)ctx->num_cus * (uint32_t)ctx->queue_occ[which];
+}
+
+/* How a batch's one-lane bins run: see slice_lanes(). */
+typedef struct {
+    uint32_t num_cands;
+    double   per_wave;      /* work of the batch's one-lane bins, in the unit of slice_lanes(), per wave that the chip
+                               holds (0: not known) */
+    int      binned;
+} slice_load_t;
+
+static slice_load_t slice_load(const myers_ctx_t *ctx, const bin_scan_t *scan, uint32_t num_queries,
+                               uint32_t num_cands, int binned)
+{
+    slice_load_t l = {num_cands, 0.0, binned};
+    if (!scan->sized || num_queries == 0) return l;
+    double work = 0.0;
+    for (uint32_t v = 0; v < ctx->num_variants; v++) {
+        const double w = (double)ctx->variants[v].words;
+        if (ctx->variants[v].lanes == 1u) work += (double)scan->reads[v] * w * w;
+    }
+    l.per_wave = work * (double)num_cands / (double)num_queries / 64.0 / (12.0 * (double)ctx->num_cus);
+    return l;
+}
+
+/* Form of the one-lane kernels for a bin of reads of up to `words` words.
+ *
+ * Chunks of 128 candidates (16 lanes per group) spend less beside the
+ * recurrence than chunks of 64 (32 lanes) but take twice as long each (about
+ * 2 words^2 in units of words^2), so a bin takes them where the batch's work
+ * is 1.5 of its chunks or more per wave (880K candidates of 100 bases: 300 us
+ * of kernels with 16 lanes, 374 with 32; 1.65M of 36-400 bases 736 us, 818
+ * with 32 lanes for all and 739 with 16 for all up to 384 bases) and the batch
+ * is large enough for the second launch (440K of 50, 100 and 150 bases: 280 us
+ * with both forms, 250 with 32 lanes).
+ *
+ * Batches that fill the chip for a few chunks only, of short reads, are bound
+ * by the latency of a chunk, which is less for the bit-vector kernel (one
+ * candidate per lane): 110K candidates of 100 bases 32 us against 41, 440K 85
+ * against 102; from 8 words on the sliced form is faster at every size (250
+ * bases, 5.5K candidates: 73 against 80 us). */
+static uint32_t slice_lanes(const myers_ctx_t *ctx, uint32_t words, const slice_load_t *l)
+{
+    const uint64_t few = (uint64_t)ctx->num_cus * (l->binned ? 1024u : 2048u);
+    if (words <= myers_slice_max_words(1u) && l->num_cands < few) return 1u;
+    const double w = (double)words;
+    return words <= myers_slice_max_words(16u) && (uint64_t)l->num_cands >= (uint64_t)ctx->num_cus * 2048u &&
+                   3.0 * w * w <= l->per_wave ? 16u : 32u;
+}
+
+/* Add variant v (one lane) to a plan of the one-lane kernel with this form. */
+static void slice_plan_add(const myers_ctx_t *ctx, myers_queue_plan_t *p, uint32_t v, uint32_t lanes)
+{
+    const uint32_t words = ctx->variants[v].words;
+    const uint32_t u4 = myers_slice_ws_u4(lanes, words);
+    p->cls = lanes == 16u ? MYERS_QUEUE_ONE_LANE_16 : MYERS_QUEUE_ONE_LANE;
+    p->variant[p->n] = v;
+    p->key[p->n] = (lanes << 8) | words;
+    p->n++;
+    if (u4 > p->ws_u4) p->ws_u4 = u4;
+}
+
+/* Launch one bin: variant v over a->start / count or its bin range, with a
+ * fixed grid (resident = 0) or a resident grid that pulls from the variant's
+ * part heads. */
+static int launch_bin(myers_ctx_t *ctx, uint32_t v, myers_verify_args_t *a, const slice_load_t *load, int resident,
+                      hipStream_t stream)
+{
+    const myers_variant_desc_t *d = &ctx->variants[v];
+    const uint32_t num_cands = load->num_cands;
+    a->variant = v;
+    a->chunk_factor = ctx->chunk_factor[v];
+    if (d->lanes == 1u) {
+        myers_queue_plan_t p;
+        memset(&p, 0, sizeof(p));
+        const uint32_t lanes = slice_lanes(ctx, d->words, load), cands = lanes == 16u ? 128u : 64u;
+        if (lanes == 1u && !resident)
+            return myers_launch_verify(v, a, grid_for(ctx, v, num_cands, a->bin_ranges != NULL), 0, stream);
+        slice_plan_add(ctx, &p, v, lanes);
+        const uint32_t chunks = (num_cands + cands - 1u) / cands;
+        const uint32_t full = queue_grid(ctx, lanes == 16u ? 2u : 3u, p.ws_u4 * 16u);
+        uint32_t grid = chunks;
+        if (a->bin_ranges && grid > full) grid = full;      /* the bin may hold any part of them */
+        return myers_launch_slice(a, &p, resident ? MYERS_SLICE_RANGES : MYERS_SLICE_PLAIN, grid, stream);
+    }
+    if (resident)
+        return myers_launch_verify(v, a, (uint32_t)ctx->num_cus * (uint32_t)ctx->occupancy_p[v], 1, stream);
+    return myers_launch_verify(v, a, grid_for(ctx, v, num_cands, a->bin_ranges != NULL), 0, stream);
 }
 
 /* Queue launches of a persistent batch: the bins (already in longest-first
  * order) of each kernel class go into one plan, in that order; bins of no
  * class (multi-lane W = 16, multi-wave variants) are left in `other`. */
-static void queue_plans(const uint32_t *bins, uint32_t n, myers_queue_plan_t *qp, uint32_t *other,
-                        uint32_t *nother)
+static void queue_plans(const myers_ctx_t *ctx, const uint32_t *bins, uint32_t n, const slice_load_t *load,
+                        myers_queue_plan_t *qp, uint32_t *other, uint32_t *nother)
 {
     memset(qp, 0, sizeof(myers_queue_plan_t) * MYERS_QUEUE_CLASSES);
     *nother = 0;
     for (uint32_t c = 0; c < (uint32_t)MYERS_QUEUE_CLASSES; c++) qp[c].cls = c;
     for (uint32_t i = 0; i < n; i++) {
         uint32_t u4 = 0;
-        const int cls = myers_variant_queue_class(bins[i], &u4);
+        int cls = myers_variant_queue_class(bins[i], &u4);
+        uint32_t lanes = 0;
+        if (cls == MYERS_QUEUE_ONE_LANE) {
+            lanes = slice_lanes(ctx, ctx->variants[bins[i]].words, load);
+            if (lanes == 16u) cls = MYERS_QUEUE_ONE_LANE_16;
+        }
         if (cls < 0 || qp[cls].n >= (uint32_t)MYERS_QUEUE_MAX) {
             other[(*nother)++] = bins[i];
             continue;
         }
         myers_queue_plan_t *q = &qp[cls];
+        if (lanes) {
+            slice_plan_add(ctx, q, bins[i], lanes);
+            continue;
+        }
         q->variant[q->n] = bins[i];
-        q->key[q->n] = 0;   /* filled by the caller from the variant table */
+        q->key[q->n] = (ctx->variants[bins[i]].lanes << 8) | ctx->variants[bins[i]].words;
         q->n++;
         if (u4 > q->ws_u4) q->ws_u4 = u4;
     }
@@ -797,6 +903,8 @@ static int enqueue_pipeline(myers_buffer_t *b, const batch_t *bt, const bin_scan
     a.ref = ctx->d_ref;
     a.ref_words = ctx->ref_words_alloc;
     a.ref_size = ctx->ref_size;
+    a.planes = ctx->d_planes;
+    a.plane_blocks = ctx->plane_blocks;
     a.peq = (const uint32_t *)bt->d_peq;
     a.qinfo = (const uint32_t *)bt->d_qinfo;
     a.num_peq_entries = bt->num_entries;
@@ -813,22 +921,33 @@ static int enqueue_pipeline(myers_buffer_t *b, const batch_t *bt, const bin_scan
     b->binned = 0;
     int rc;
     if (bt->num_cands == 0) return MYERS_SUCCESS;
-    if (engine == MYERS_ENGINE_PLAIN && scan->num_present == 1 && !scan->too_long) {
+    const int one_bin = engine == MYERS_ENGINE_PLAIN && scan->num_present == 1 && !scan->too_long;
+    const slice_load_t load = slice_load(ctx, scan, bt->num_queries, bt->num_cands, !one_bin);
+    if (one_bin) {
         const uint32_t v = scan->single;
         a.start = 0;
         a.count = bt->num_cands;
-        rc = myers_launch_verify(v, &a, grid_for(ctx, v, bt->num_cands, 0), 0, b->stream);
+        rc = launch_bin(ctx, v, &a, &load, 0, b->stream);
         if (rc) return hip_fail((hipError_t)rc, "verify launch", __FILE__, __LINE__);
         b->stats.launches = 1;
         b->stats.variantsUsed = 1;
         return MYERS_SUCCESS;
     }
-    /* Threshold mode: the band probe classes the candidates of one-lane
-     * cut-off variants (before the binning) and orders their bins (after). */
-    const uint64_t probe = bt->threshold >= 0.0f ? ctx->probe_mask & scan->present : 0u;
-    if (probe) {
-        rc = myers_launch_probe(&a, bt->num_cands, ctx->d_bin_of_words, max_supported_words(ctx), probe, b->stream);
-        if (rc) return hip_fail((hipError_t)rc, "probe launch", __FILE__, __LINE__);
+    /* Chunks of the sliced kernels with an N in some read run slower; in a
+     * large batch the candidates of such reads are put together.  The two
+     * passes take about 12 us per million candidates, which pays where the
+     * chunks are long: bins of over GROUP_N_WORDS words, in batches whose
+     * one-lane reads average that (1000 bases: 7.08 -> 6.7 ms; 100 bases, if it
+     * were done: 1.02 -> 1.10 ms). */
+    uint64_t group_n = 0;
+    if ((uint64_t)bt->num_cands >= 1024u * (uint64_t)ctx->num_cus &&
+        load.per_wave * 64.0 * 12.0 * (double)ctx->num_cus >= (double)(GROUP_N_WORDS * GROUP_N_WORDS) * (double)bt->num_cands) {
+        for (uint32_t v = 0; v < ctx->num_variants; v++)
+            if (ctx->variants[v].lanes == 1u && ctx->variants[v].words > GROUP_N_WORDS) group_n |= scan->present & (1ull << v);
+    }
+    if (group_n) {
+        rc = myers_launch_read_n(&a, bt->num_cands, 32u * GROUP_N_WORDS, 32u * myers_slice_max_words(32u), b->stream);
+        if (rc) return hip_fail((hipError_t)rc, "read N launch", __FILE__, __LINE__);
     }
     /* device-side binning */
     uint32_t *ranges = bt->d_work + MYERS_WORK_RANGES;
@@ -839,10 +958,10 @@ static int enqueue_pipeline(myers_buffer_t *b, const batch_t *bt, const bin_scan
                               bt->d_work + MYERS_WORK_BLOCKS, ranges, bt->d_order, err, bt->d_results, heads,
                               b->stream);
     if (rc) return hip_fail((hipError_t)rc, "binning launch", __FILE__, __LINE__);
-    if (probe) {
-        rc = myers_launch_probe_order(ranges, ctx->num_variants, probe, bt->num_cands, bt->d_order, bt->d_results,
-                                      b->stream);
-        if (rc) return hip_fail((hipError_t)rc, "probe order launch", __FILE__, __LINE__);
+    if (group_n) {
+        rc = myers_launch_group_n(ranges, ctx->num_variants, group_n, bt->num_cands, bt->d_order, bt->d_results,
+                                  b->stream);
+        if (rc) return hip_fail((hipError_t)rc, "group N launch", __FILE__, __LINE__);
     }
     HIP_TRY(hipMemcpyAsync(b->h_err, err, sizeof(uint32_t), hipMemcpyDeviceToHost, b->stream));
     if (b->mark_slot >= 0) {
@@ -860,8 +979,7 @@ static int enqueue_pipeline(myers_buffer_t *b, const batch_t *bt, const bin_scan
     if (engine == MYERS_ENGINE_PLAIN) {
         /* one launch per length bin, in turn */
         for (uint32_t i = 0; i < n; i++) {
-            a.variant = order[i];
-            rc = myers_launch_verify(order[i], &a, grid_for(ctx, order[i], bt->num_cands, 1), 0, b->stream);
+            rc = launch_bin(ctx, order[i], &a, &load, 0, b->stream);
             if (rc) return hip_fail((hipError_t)rc, "verify launch", __FILE__, __LINE__);
         }
     } else {
@@ -887,12 +1005,8 @@ static int enqueue_pipeline(myers_buffer_t *b, const batch_t *bt, const bin_scan
         myers_queue_plan_t qp[MYERS_QUEUE_CLASSES];
         uint32_t other[MYERS_MAX_VARIANTS], nother = 0, nqueue = 0;
         if (engine == MYERS_ENGINE_PERSISTENT) {
-            queue_plans(rest, nrest, qp, other, &nother);
-            for (uint32_t c = 0; c < (uint32_t)MYERS_QUEUE_CLASSES; c++) {
-                for (uint32_t j = 0; j < qp[c].n; j++)
-                    qp[c].key[j] = (ctx->variants[qp[c].variant[j]].lanes << 8) | ctx->variants[qp[c].variant[j]].words;
-                nqueue += qp[c].n ? 1u : 0u;
-            }
+            queue_plans(ctx, rest, nrest, &load, qp, other, &nother);
+            for (uint32_t c = 0; c < (uint32_t)MYERS_QUEUE_CLASSES; c++) nqueue += qp[c].n ? 1u : 0u;
         } else {
             memset(qp, 0, sizeof(qp));
             memcpy(other, rest, nrest * sizeof(uint32_t));
@@ -918,16 +1032,15 @@ static int enqueue_pipeline(myers_buffer_t *b, const batch_t *bt, const bin_scan
         }
         for (uint32_t c = 0; c < (uint32_t)MYERS_QUEUE_CLASSES; c++) {
             if (qp[c].n == 0) continue;
-            const int cut = bt->threshold >= 0.0f;
-            rc = myers_launch_queue(&a, &qp[c], queue_grid(ctx, c, cut, qp[c].ws_u4 * 16u), NEXT_STREAM());
+            const int multi = c == MYERS_QUEUE_MULTI_LANE;
+            const uint32_t which = !multi ? (c == MYERS_QUEUE_ONE_LANE_16 ? 2u : 3u) : (bt->threshold >= 0.0f ? 1u : 0u);
+            const uint32_t grid = queue_grid(ctx, which, qp[c].ws_u4 * 16u);
+            rc = multi ? myers_launch_queue(&a, &qp[c], grid, NEXT_STREAM())
+                       : myers_launch_slice(&a, &qp[c], MYERS_SLICE_QUEUE, grid, NEXT_STREAM());
             if (rc) return hip_fail((hipError_t)rc, "queue launch", __FILE__, __LINE__);
         }
         for (uint32_t i = 0; i < nother; i++) {
-            const uint32_t v = other[i];
-            a.variant = v;
-            a.chunk_factor = ctx->chunk_factor[v];
-            uint64_t grid = (uint64_t)ctx->num_cus * (uint64_t)ctx->occupancy_p[v];
-            rc = myers_launch_verify(v, &a, (uint32_t)grid, 1, NEXT_STREAM());
+            rc = launch_bin(ctx, other[i], &a, &load, 1, NEXT_STREAM());
             if (rc) return hip_fail((hipError_t)rc, "persistent launch", __FILE__, __LINE__);
         }
 #undef NEXT_STREAM

@@ -34,6 +34,8 @@ typedef struct {
     const uint32_t *ref;         /* packed reference + guard words (all-N) */
     uint64_t        ref_words;   /* words readable at ref (incl. guard) */
     uint64_t        ref_size;    /* reference length in bases */
+    const uint32_t *planes;      /* its bit planes, 3 words per 32 bases (one-lane variants) */
+    uint32_t        plane_blocks;
     const uint32_t *peq;         /* qryEntry_t[] as u32[20] */
     const uint32_t *qinfo;       /* qryInfo_t[] as u32 pairs {posEntry, size} */
     uint32_t        num_peq_entries;
@@ -47,8 +49,8 @@ typedef struct {
     uint32_t        mode;        /* 0 aligned window, 1 exact-start window */
     float           distance;
     float           threshold;   /* < 0: off; else results above (uint32)(m*threshold) get
-                                    {0xFFFFFFFF, 0xFFFFFFFF}; L = 1 variants cut off rows and
-                                    L = 4..64 variants stop hopeless waves */
+                                    {0xFFFFFFFF, 0xFFFFFFFF}; L = 4..64 variants stop hopeless
+                                    waves */
     uint32_t        chunk_factor;  /* persistent launch: chunks per queue pull */
     void           *results;     /* resEntry_t[] in caller order */
     uint32_t       *queue_heads; /* persistent launch: MYERS_QUEUE_WORDS words of part heads */
@@ -114,34 +116,56 @@ int myers_launch_long(const myers_verify_args_t *args, const myers_long_plan_t *
  * reads first, so the tail is short chunks); each chunk runs the variant of
  * its bin through a switch over the compiled variants.  Variants fall into
  * two kernel classes with their own register budgets: MYERS_QUEUE_ONE_LANE
- * (L = 1; one-wave workgroups, one chunk per item) and MYERS_QUEUE_MULTI_LANE
- * (L = 2..64 with W <= 12; workgroups of myers_queue_waves() = 2 waves that
- * take a pair of chunks per item and share one staged Peq, so that each wave
- * needs half the LDS); other variants keep per-bin launches.  The class's
+ * (L = 1: the candidate-sliced kernel, below) and MYERS_QUEUE_MULTI_LANE
+ * (L = 2..64 with W <= 12; workgroups of two waves that take a pair of chunks
+ * per item and share one staged Peq, so that each wave needs half the LDS);
+ * other variants keep per-bin launches.  The class's
  * counter (queue_heads + MYERS_QUEUE_HEAD(cls)) is reset by the binning.
  * LDS per workgroup: ws_u4 x 16 bytes (the largest workspace of the plan's
- * variants, as myers_variant_queue_class reports it).  Needs bin_ranges and
- * queue_heads. */
-enum { MYERS_QUEUE_ONE_LANE = 0, MYERS_QUEUE_MULTI_LANE = 1, MYERS_QUEUE_CLASSES = 2, MYERS_QUEUE_MAX = 48 };
+ * variants, as myers_variant_queue_class or myers_slice_ws_u4 reports it).
+ * Needs bin_ranges and queue_heads. */
+enum { MYERS_QUEUE_ONE_LANE = 0, MYERS_QUEUE_MULTI_LANE = 1, MYERS_QUEUE_ONE_LANE_16 = 2, MYERS_QUEUE_CLASSES = 3,
+       MYERS_QUEUE_MAX = 48 };
 #define MYERS_QUEUE_HEAD(cls) (MYERS_LONG_HEAD + (2u + (uint32_t)(cls)) * MYERS_QUEUE_STRIDE)
 typedef struct {
-    uint32_t cls;                        /* MYERS_QUEUE_ONE_LANE or MYERS_QUEUE_MULTI_LANE */
+    uint32_t cls;                        /* MYERS_QUEUE_MULTI_LANE, MYERS_QUEUE_ONE_LANE (32 lanes per
+                                            group) or MYERS_QUEUE_ONE_LANE_16 */
     uint32_t n;                          /* bins, in pull order */
     uint32_t ws_u4;                      /* LDS per workgroup in 16-byte units */
     uint32_t reserved;
     uint32_t variant[MYERS_QUEUE_MAX];   /* variant ids (rows of bin_ranges) */
-    uint32_t key[MYERS_QUEUE_MAX];       /* lanes << 8 | words of each */
+    uint32_t key[MYERS_QUEUE_MAX];       /* lanes << 8 | words of each; one-lane class: the
+                                            lanes of its sliced form */
 } myers_queue_plan_t;
-/* Class of variant v in the queue launch (-1: none) and its workspace. */
+/* Class of variant v in the queue launch (-1: none) and, for the multi-lane
+ * class, its workspace. */
 int myers_variant_queue_class(uint32_t v, uint32_t *ws_u4);
-/* Resident workgroups per CU of a class's queue kernel with `lds_bytes` of
- * dynamic LDS (cut: the threshold-mode kernel). */
-int myers_queue_occupancy(uint32_t cls, int cut, uint32_t lds_bytes, int *wg_per_cu);
-/* Waves per workgroup of a class's queue kernel. */
-uint32_t myers_queue_waves(uint32_t cls);
-/* grid = workgroups (normally CUs x occupancy). */
+/* Resident workgroups per CU of the multi-lane queue kernel with `lds_bytes`
+ * of dynamic LDS (cut: the threshold-mode kernel). */
+int myers_queue_occupancy(int cut, uint32_t lds_bytes, int *wg_per_cu);
+/* Multi-lane plans; grid = workgroups (normally CUs x occupancy). */
 int myers_launch_queue(const myers_verify_args_t *args, const myers_queue_plan_t *plan, uint32_t grid,
                        hipStream_t stream);
+
+/* One-lane variants (reads of up to 1024 bases) run the candidate-sliced
+ * kernel (myers_slice.h), which has a form of 16 and one of 32 lanes per group
+ * of 32 candidates: a one-wave workgroup takes 2048 / lanes candidates of one
+ * bin, reads of up to myers_slice_max_words(lanes) words.  Form 1 is the
+ * bit-vector kernel (chunks of 64).  A plan holds bins of form 16, or of forms
+ * 1 and 32; modes: every bin from the queue counter, or a plan of
+ * one bin with a fixed grid over args->start / count or its bin range
+ * (MYERS_SLICE_PLAIN) or a resident grid pulling guided ranges of at least
+ * chunk_factor chunks from the variant's part heads (MYERS_SLICE_RANGES). */
+enum { MYERS_SLICE_PLAIN = 0, MYERS_SLICE_RANGES = 1, MYERS_SLICE_QUEUE = 2 };
+uint32_t myers_slice_max_words(uint32_t lanes);
+uint32_t myers_slice_ws_u4(uint32_t lanes, uint32_t words);     /* LDS in 16-byte units, 0: no such form */
+int myers_slice_occupancy(uint32_t lanes, uint32_t lds_bytes, int *wg_per_cu);
+int myers_launch_slice(const myers_verify_args_t *args, const myers_queue_plan_t *plan, uint32_t mode, uint32_t grid,
+                       hipStream_t stream);
+/* Bit planes of the packed reference (3 words per block of 32 bases, the
+ * last block padded with N). */
+int myers_launch_planes(const uint32_t *ref, uint64_t ref_words, uint32_t *planes, uint32_t nblocks,
+                        hipStream_t stream);
 
 /* Resident serving kernel.  A grid of one-wave workgroups stays on the
  * device and verifies work items published by a host thread: each item is a
@@ -268,27 +292,15 @@ int myers_launch_binning(const uint32_t *qinfo, uint32_t num_queries, const void
                          uint32_t *block_counts, uint32_t *ranges, uint32_t *order, uint32_t *err,
                          void *results, uint32_t *queue_heads, hipStream_t stream);
 
-/* Threshold mode's band probe.  The cut-off advances a wave of one-lane
- * candidates as deep as its deepest lane, and a candidate whose read occurs
- * in its window keeps most of the column's rows within the threshold; in a
- * batch where such candidates are spread over every wave, every wave runs
- * deep.  myers_launch_probe (before the binning) classes every candidate
- * whose variant v has bit v set in probe_mask: the first 32 bases of the read
- * (one bit-vector word) run over the leading min(n, 2 d m + 72) columns of
- * its window, where a read placed by the filter begins, and results[i].x
- * gets 0 when some column has D <= 8 there, else 1; other candidates get 0.
- * The args' peq, qinfo, cands, ref, mode, distance and results are used.
- * myers_launch_probe_order (after the binning) reorders each probed
- * variant's range in spans of two 64-slot chunks so that the first chunk
- * takes the span's class-0 candidates (then class 1 in slot order), keeping
- * a read's candidates in runs.  Both only order the work: the results are
- * those of the batch without them. */
-int myers_launch_probe(const myers_verify_args_t *args, uint32_t num_cands, const uint8_t *bin_of_words,
-                       uint32_t max_words, uint64_t probe_mask, hipStream_t stream);
-int myers_launch_probe_order(const uint32_t *ranges, uint32_t num_variants, uint64_t probe_mask,
-                             uint32_t num_cands, uint32_t *order, const void *results, hipStream_t stream);
-/* The variants worth probing: one-lane variants with a cut-off kernel. */
-uint64_t myers_probe_variants(void);
+/* Candidates of reads with an N put together (order of the work only; the
+ * results stay in the caller's order): read_n, before the binning, leaves in
+ * results[i].x whether candidate i's read (of min_m to max_m bases) holds an N;
+ * group_n, after it, moves those candidates to the front of each span of slots
+ * of the ranges of the variants with their bit in `variants` set. */
+int myers_launch_read_n(const myers_verify_args_t *args, uint32_t num_cands, uint32_t min_m, uint32_t max_m,
+                        hipStream_t stream);
+int myers_launch_group_n(const uint32_t *ranges, uint32_t num_variants, uint64_t variants, uint32_t num_cands,
+                         uint32_t *order, const void *results, hipStream_t stream);
 
 #ifdef __cplusplus
 }
