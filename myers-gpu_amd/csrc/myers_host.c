@@ -103,7 +103,7 @@ typedef struct myers_buffer {
     hipEvent_t   ev_fork, ev_join[SIDE_STREAMS];
     /* steady-state graph of the last device-resident batch shape */
     hipGraphExec_t graph_exec;
-    uint64_t     graph_key[12];
+    uint64_t     graph_key[13];
     int          graph_valid;
     int          graph_binned;
     uint32_t     graph_launches;
@@ -832,6 +832,52 @@ static void slice_plan_add(const myers_ctx_t *ctx, myers_queue_plan_t *p, uint32
     if (u4 > p->ws_u4) p->ws_u4 = u4;
 }
 
+/* The bins of a batch whose reads of over 1024 bases run the sliced kernel
+ * (myers_launch_wide_slice): all of them, or none.
+ *
+ * That kernel has about 1.6 times the rate of the multi-lane bit-vector
+ * kernels, but a chunk of 32 candidates takes as long as many rounds of
+ * theirs, so it pays where the batch fills the chip with chunks.  Both times
+ * are estimated, a bin's mean read counting 0.8 of its longest: a step of 12
+ * waves costs 28 ns per row of a lane and 60 ns beside (T waves per chunk, steps
+ * for 1.25 m columns and the lag over the waves) and the last chunks leave 0.4
+ * of one chunk's time idle; the bit-vector kernels run 120e12 cells per second behind one candidate's chain.  1000-4000
+ * bases, 4 candidates each: 16,000 reads 3.9 ms against 5.4 bit-vector, 8,000
+ * reads 3.8 against 3.1; 2-20 kb: 20,000 reads 46 against 68, 6,400 reads 22.6
+ * and 22.6, 3,200 reads 22.1 against 12.5. */
+static uint64_t wide_bins(const myers_ctx_t *ctx, const bin_scan_t *scan, const batch_t *bt)
+{
+    const uint32_t engine = bt->flags & MYERS_ENGINE_MASK;
+    if (!scan->sized || scan->too_long || bt->num_queries == 0 || bt->threshold >= 0.0f ||
+        (engine != MYERS_ENGINE_AUTO && engine != MYERS_ENGINE_PERSISTENT))
+        return 0;
+    const double cpr = (double)bt->num_cands / (double)bt->num_queries;
+    uint64_t mask = 0;
+    double cells = 0.0, old_chain = 0.0, work = 0.0, longest = 0.0;      /* times in ns */
+    for (uint32_t v = 0; v < ctx->num_variants; v++) {
+        const myers_variant_desc_t *d = &ctx->variants[v];
+        if (!(scan->present & (1ull << v)) || d->lanes == 1u) continue;
+        const uint32_t team = myers_wide_slice_team(d->total_words);
+        const double cands = scan->counted ? (double)scan->cands[v] : (double)scan->reads[v] * cpr;
+        if (team == 0u) return 0;
+        if (cands <= 0.0) continue;
+        const double m = (double)scan->max_m[v];
+        const double rows = (double)((scan->max_m[v] + 64u * team - 1u) / (64u * team));
+        const double chunk = (1.25 * m + 96.0 * team) * (60.0 + 28.0 * rows);
+        const uint32_t four = 64u * MYERS_LONG_WAVES;
+        const double chain = d->total_words > four
+                                 ? chain_ns(scan->max_m[v], four, (d->total_words + four - 1u) / four, 1)
+                                 : chain_ns(scan->max_m[v], d->lanes, d->words, 0);
+        work += (1.0 + 0.8 * cands / (32.0 * (MYERS_WIDE_SLICE_WAVES / team))) * chunk;
+        cells += 0.8 * cands * 1.25 * m * m;
+        if (chunk > longest) longest = chunk;
+        if (chain > old_chain) old_chain = chain;
+        mask |= 1ull << v;
+    }
+    const double wide = work / (double)ctx->num_cus + 0.4 * longest;
+    return (wide > longest ? wide : longest) < cells / 120e3 + old_chain ? mask : 0;
+}
+
 /* Launch one bin: variant v over a->start / count or its bin range, with a
  * fixed grid (resident = 0) or a resident grid that pulls from the variant's
  * part heads. */
@@ -864,7 +910,7 @@ static int launch_bin(myers_ctx_t *ctx, uint32_t v, myers_verify_args_t *a, cons
  * order) of each kernel class go into one plan, in that order; bins of no
  * class (multi-lane W = 16, multi-wave variants) are left in `other`. */
 static void queue_plans(const myers_ctx_t *ctx, const uint32_t *bins, uint32_t n, const slice_load_t *load,
-                        myers_queue_plan_t *qp, uint32_t *other, uint32_t *nother)
+                        uint64_t wide, myers_queue_plan_t *qp, uint32_t *other, uint32_t *nother)
 {
     memset(qp, 0, sizeof(myers_queue_plan_t) * MYERS_QUEUE_CLASSES);
     *nother = 0;
@@ -877,6 +923,7 @@ static void queue_plans(const myers_ctx_t *ctx, const uint32_t *bins, uint32_t n
             lanes = slice_lanes(ctx, ctx->variants[bins[i]].words, load);
             if (lanes == 16u) cls = MYERS_QUEUE_ONE_LANE_16;
         }
+        if ((wide >> bins[i]) & 1ull) cls = MYERS_QUEUE_WIDE;
         if (cls < 0 || qp[cls].n >= (uint32_t)MYERS_QUEUE_MAX) {
             other[(*nother)++] = bins[i];
             continue;
@@ -887,7 +934,8 @@ static void queue_plans(const myers_ctx_t *ctx, const uint32_t *bins, uint32_t n
             continue;
         }
         q->variant[q->n] = bins[i];
-        q->key[q->n] = (ctx->variants[bins[i]].lanes << 8) | ctx->variants[bins[i]].words;
+        q->key[q->n] = cls == MYERS_QUEUE_WIDE ? myers_wide_slice_team(ctx->variants[bins[i]].total_words)
+                                               : (ctx->variants[bins[i]].lanes << 8) | ctx->variants[bins[i]].words;
         q->n++;
         if (u4 > q->ws_u4) q->ws_u4 = u4;
     }
@@ -915,7 +963,8 @@ static int enqueue_pipeline(myers_buffer_t *b, const batch_t *bt, const bin_scan
     a.threshold = bt->threshold;
     a.results = bt->d_results;
 
-    const uint32_t engine = resolve_engine(ctx, bt->flags, scan, bt->num_cands);
+    const uint64_t wide = wide_bins(ctx, scan, bt);
+    const uint32_t engine = wide ? (uint32_t)MYERS_ENGINE_PERSISTENT : resolve_engine(ctx, bt->flags, scan, bt->num_cands);
     b->stats.launches = 0;
     b->stats.variantsUsed = 0;
     b->binned = 0;
@@ -945,8 +994,9 @@ static int enqueue_pipeline(myers_buffer_t *b, const batch_t *bt, const bin_scan
         for (uint32_t v = 0; v < ctx->num_variants; v++)
             if (ctx->variants[v].lanes == 1u && ctx->variants[v].words > GROUP_N_WORDS) group_n |= scan->present & (1ull << v);
     }
-    if (group_n) {
-        rc = myers_launch_read_n(&a, bt->num_cands, 32u * GROUP_N_WORDS, 32u * myers_slice_max_words(32u), b->stream);
+    if (group_n || wide) {
+        rc = myers_launch_read_n(&a, bt->num_cands, group_n ? 32u * GROUP_N_WORDS : 32u * myers_slice_max_words(32u),
+                                 wide ? ~0u : 32u * myers_slice_max_words(32u), b->stream);
         if (rc) return hip_fail((hipError_t)rc, "read N launch", __FILE__, __LINE__);
     }
     /* device-side binning */
@@ -962,6 +1012,10 @@ static int enqueue_pipeline(myers_buffer_t *b, const batch_t *bt, const bin_scan
         rc = myers_launch_group_n(ranges, ctx->num_variants, group_n, bt->num_cands, bt->d_order, bt->d_results,
                                   b->stream);
         if (rc) return hip_fail((hipError_t)rc, "group N launch", __FILE__, __LINE__);
+    }
+    if (wide) {
+        rc = myers_launch_sort_len(&a, ranges, ctx->num_variants, wide, bt->num_cands, bt->d_order, b->stream);
+        if (rc) return hip_fail((hipError_t)rc, "sort launch", __FILE__, __LINE__);
     }
     HIP_TRY(hipMemcpyAsync(b->h_err, err, sizeof(uint32_t), hipMemcpyDeviceToHost, b->stream));
     if (b->mark_slot >= 0) {
@@ -993,7 +1047,7 @@ static int enqueue_pipeline(myers_buffer_t *b, const batch_t *bt, const bin_scan
          * others. */
         myers_long_plan_t lp;
         uint32_t nlong = 0;
-        if (bt->flags & MYERS_NO_LONG_LAUNCH) memset(&lp, 0, sizeof(lp));
+        if (wide || (bt->flags & MYERS_NO_LONG_LAUNCH)) memset(&lp, 0, sizeof(lp));
         else nlong = long_plan(ctx, scan, bt, order, n, &lp);
         uint32_t rest[MYERS_MAX_VARIANTS], nrest = 0;
         for (uint32_t i = 0; i < n; i++) {
@@ -1005,7 +1059,7 @@ static int enqueue_pipeline(myers_buffer_t *b, const batch_t *bt, const bin_scan
         myers_queue_plan_t qp[MYERS_QUEUE_CLASSES];
         uint32_t other[MYERS_MAX_VARIANTS], nother = 0, nqueue = 0;
         if (engine == MYERS_ENGINE_PERSISTENT) {
-            queue_plans(ctx, rest, nrest, &load, qp, other, &nother);
+            queue_plans(ctx, rest, nrest, &load, wide, qp, other, &nother);
             for (uint32_t c = 0; c < (uint32_t)MYERS_QUEUE_CLASSES; c++) nqueue += qp[c].n ? 1u : 0u;
         } else {
             memset(qp, 0, sizeof(qp));
@@ -1030,8 +1084,15 @@ static int enqueue_pipeline(myers_buffer_t *b, const batch_t *bt, const bin_scan
             rc = myers_launch_long(&a, &lp, ctx->num_cus, NEXT_STREAM());
             if (rc) return hip_fail((hipError_t)rc, "long-read launch", __FILE__, __LINE__);
         }
-        for (uint32_t c = 0; c < (uint32_t)MYERS_QUEUE_CLASSES; c++) {
+        /* (longest reads first) */
+        for (uint32_t k = 0; k < (uint32_t)MYERS_QUEUE_CLASSES; k++) {
+            const uint32_t c = (k + (uint32_t)MYERS_QUEUE_WIDE) % (uint32_t)MYERS_QUEUE_CLASSES;
             if (qp[c].n == 0) continue;
+            if (c == MYERS_QUEUE_WIDE) {
+                rc = myers_launch_wide_slice(&a, &qp[c], ctx->num_cus, NEXT_STREAM());
+                if (rc) return hip_fail((hipError_t)rc, "queue launch", __FILE__, __LINE__);
+                continue;
+            }
             const int multi = c == MYERS_QUEUE_MULTI_LANE;
             const uint32_t which = !multi ? (c == MYERS_QUEUE_ONE_LANE_16 ? 2u : 3u) : (bt->threshold >= 0.0f ? 1u : 0u);
             const uint32_t grid = queue_grid(ctx, which, qp[c].ws_u4 * 16u);
@@ -1114,12 +1175,13 @@ static int enqueue_verify(myers_buffer_t *b, const batch_t *bt, const qryInfo_t 
                               ((uint64_t)long_plan(b->ctx, &scan, bt, order,
                                                    present_by_cost(b->ctx, scan.present, order), &lp) |
                                ((uint64_t)lp.n_wide << 32));
-    const uint64_t key[12] = {(uint64_t)(uintptr_t)bt->d_peq, (uint64_t)(uintptr_t)bt->d_qinfo,
+    const uint64_t key[13] = {(uint64_t)(uintptr_t)bt->d_peq, (uint64_t)(uintptr_t)bt->d_qinfo,
                               (uint64_t)(uintptr_t)bt->d_cands, (uint64_t)(uintptr_t)bt->d_results,
                               ((uint64_t)bt->num_entries << 32) | bt->num_queries,
                               ((uint64_t)bt->num_cands << 32) | bt->flags,
                               (uint64_t)dist_bits, scan.present,
-                              (uint64_t)scan.too_long, b->ctx->tune_gen, (uint64_t)thr_bits, plan_key};
+                              (uint64_t)scan.too_long, b->ctx->tune_gen, (uint64_t)thr_bits, plan_key,
+                              wide_bins(b->ctx, &scan, bt)};
     if (!b->graph_valid || memcmp(key, b->graph_key, sizeof(key)) != 0) {
         if (b->graph_exec) {
             hipGraphExecDestroy(b->graph_exec);

@@ -124,8 +124,8 @@ int myers_launch_long(const myers_verify_args_t *args, const myers_long_plan_t *
  * LDS per workgroup: ws_u4 x 16 bytes (the largest workspace of the plan's
  * variants, as myers_variant_queue_class or myers_slice_ws_u4 reports it).
  * Needs bin_ranges and queue_heads. */
-enum { MYERS_QUEUE_ONE_LANE = 0, MYERS_QUEUE_MULTI_LANE = 1, MYERS_QUEUE_ONE_LANE_16 = 2, MYERS_QUEUE_CLASSES = 3,
-       MYERS_QUEUE_MAX = 48 };
+enum { MYERS_QUEUE_ONE_LANE = 0, MYERS_QUEUE_MULTI_LANE = 1, MYERS_QUEUE_ONE_LANE_16 = 2, MYERS_QUEUE_WIDE = 3,
+       MYERS_QUEUE_CLASSES = 4, MYERS_QUEUE_MAX = 48 };
 #define MYERS_QUEUE_HEAD(cls) (MYERS_LONG_HEAD + (2u + (uint32_t)(cls)) * MYERS_QUEUE_STRIDE)
 typedef struct {
     uint32_t cls;                        /* MYERS_QUEUE_MULTI_LANE, MYERS_QUEUE_ONE_LANE (32 lanes per
@@ -162,6 +162,15 @@ uint32_t myers_slice_ws_u4(uint32_t lanes, uint32_t words);     /* LDS in 16-byt
 int myers_slice_occupancy(uint32_t lanes, uint32_t lds_bytes, int *wg_per_cu);
 int myers_launch_slice(const myers_verify_args_t *args, const myers_queue_plan_t *plan, uint32_t mode, uint32_t grid,
                        hipStream_t stream);
+/* Multi-lane variants in large batches (threshold mode off): the
+ * candidate-sliced recurrence on workgroups of MYERS_WIDE_SLICE_WAVES waves, one
+ * per CU, in teams that take 32 candidates each (myers_slice_wide.hip); bins
+ * ordered by myers_launch_sort_len first.  Plans of class MYERS_QUEUE_WIDE: key
+ * is the waves per team that myers_wide_slice_team says (0: reads too long). */
+enum { MYERS_WIDE_SLICE_WAVES = 12 };
+uint32_t myers_wide_slice_team(uint32_t words);
+int myers_launch_wide_slice(const myers_verify_args_t *args, const myers_queue_plan_t *plan, uint32_t grid,
+                            hipStream_t stream);
 /* Bit planes of the packed reference (3 words per block of 32 bases, the
  * last block padded with N). */
 int myers_launch_planes(const uint32_t *ref, uint64_t ref_words, uint32_t *planes, uint32_t nblocks,
@@ -301,6 +310,11 @@ int myers_launch_read_n(const myers_verify_args_t *args, uint32_t num_cands, uin
                         hipStream_t stream);
 int myers_launch_group_n(const uint32_t *ranges, uint32_t num_variants, uint64_t variants, uint32_t num_cands,
                          uint32_t *order, const void *results, hipStream_t stream);
+/* Order each span of 4096 slots of the bins in `variants`: candidates of reads
+ * with N (as myers_launch_read_n left it in the results) first, then by read
+ * length, longest first; candidates of one read stay together. */
+int myers_launch_sort_len(const myers_verify_args_t *args, const uint32_t *ranges, uint32_t num_variants,
+                          uint64_t variants, uint32_t num_cands, uint32_t *order, hipStream_t stream);
 
 #ifdef __cplusplus
 }

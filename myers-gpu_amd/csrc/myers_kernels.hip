@@ -799,6 +799,57 @@ __global__ __launch_bounds__(256) void group_n_kernel(const uint32_t *ranges, ui
     }
 }
 
+// Sort each span of kLenSpan slots of a variant's range: reads with N first
+// (read_n_kernel), then by read length, longest first, then by slot (so a
+// read's candidates stay together).  A bitonic network over keys of the three
+// in LDS, one block per span.
+constexpr uint32_t kLenSpan = 4096u;
+__global__ __launch_bounds__(1024) void sort_len_kernel(myers_verify_args_t a, const uint32_t *ranges, uint32_t nv,
+                                                        uint64_t mask, uint32_t *order) {
+    __shared__ uint32_t key[kLenSpan], cand[kLenSpan];
+    uint32_t spans = 0;                                 // of the variants before v
+    for (uint32_t v = 0; v < nv && v < 64u; v++) {
+        if (!((mask >> v) & 1ull)) continue;
+        const uint32_t start = ranges[2 * v], count = ranges[2 * v + 1];
+        const uint32_t here = (count + kLenSpan - 1u) / kLenSpan;
+        // block b takes the spans b, b + gridDim, .. of all variants' spans
+        const uint32_t skip = (blockIdx.x + gridDim.x - spans % gridDim.x) % gridDim.x;
+        for (uint32_t sp = skip; sp < here; sp += gridDim.x) {
+            const uint32_t s0 = start + sp * kLenSpan, len = min(kLenSpan, count - sp * kLenSpan);
+            uint32_t n = 2;                             // keys sorted: a power of two
+            while (n < len) n *= 2u;
+            __syncthreads();                            // the previous span is written
+            for (uint32_t at = threadIdx.x; at < n; at += 1024u) {
+                uint32_t k = ~0u;
+                if (at < len) {
+                    const uint32_t c = order[s0 + at], query = static_cast<const CandRec *>(a.cands)[c].query;
+                    const uint32_t m = query < a.num_queries ? reinterpret_cast<const uint2 *>(a.qinfo)[query].y : 0u;
+                    cand[at] = c;
+                    const uint32_t n_last = static_cast<const uint2 *>(a.results)[c].x & 1u ? 0u : 1u << 31;
+                    k = n_last | ((0x7FFFFu - min(m, 0x7FFFFu)) << 12) | at;
+                }
+                key[at] = k;
+            }
+            __syncthreads();
+            for (uint32_t size = 2; size <= n; size *= 2u) {
+                for (uint32_t d = size / 2u; d > 0u; d /= 2u) {
+                    for (uint32_t i = threadIdx.x; i < n / 2u; i += 1024u) {
+                        const uint32_t lo = 2u * i - (i & (d - 1u)), hi = lo + d;
+                        const uint32_t x = key[lo], y = key[hi];
+                        if ((x > y) == ((lo & size) == 0u)) {
+                            key[lo] = y;
+                            key[hi] = x;
+                        }
+                    }
+                    __syncthreads();
+                }
+            }
+            for (uint32_t at = threadIdx.x; at < len; at += 1024u) order[s0 + at] = cand[key[at] & (kLenSpan - 1u)];
+        }
+        spans += here;
+    }
+}
+
 }  // namespace
 
 // ------------------------------------------------------------ variant table
@@ -1065,5 +1116,15 @@ extern "C" int myers_launch_group_n(const uint32_t *ranges, uint32_t num_variant
     if (grid > 2048u) grid = 2048u;
     hipLaunchKernelGGL(group_n_kernel, dim3(grid), dim3(256), 0, stream, ranges, num_variants, variants, order,
                        static_cast<const uint2 *>(results));
+    return (int)hipGetLastError();
+}
+
+extern "C" int myers_launch_sort_len(const myers_verify_args_t *args, const uint32_t *ranges, uint32_t num_variants,
+                                     uint64_t variants, uint32_t num_cands, uint32_t *order, hipStream_t stream) {
+    if (args == nullptr || ranges == nullptr || order == nullptr || num_variants > MYERS_MAX_VARIANTS) return -1;
+    uint32_t grid = num_cands / kLenSpan + (uint32_t)__builtin_popcountll(variants);
+    if (grid > 1024u) grid = 1024u;
+    if (grid == 0u) return 0;
+    hipLaunchKernelGGL(sort_len_kernel, dim3(grid), dim3(1024), 0, stream, *args, ranges, num_variants, variants, order);
     return (int)hipGetLastError();
 }
