@@ -59,6 +59,7 @@ typedef struct myers_ctx {
     myers_variant_desc_t variants[MYERS_MAX_VARIANTS];
     int       occupancy[MYERS_MAX_VARIANTS];       /* plain kernel, workgroups per CU */
     int       occupancy_p[MYERS_MAX_VARIANTS];     /* persistent kernel */
+    uint64_t  multi_lane, deep;   /* masks: variants of several lanes; one-lane ones of 8 words or more */
     uint32_t  chunk_factor[MYERS_MAX_VARIANTS];    /* persistent: chunks per queue pull */
     uint32_t  long_seq;                            /* long-read launches so far (placement rotation) */
     int       queue_occ[4];                        /* workgroups per CU of the multi-lane queue kernel, its
@@ -103,7 +104,7 @@ typedef struct myers_buffer {
     hipEvent_t   ev_fork, ev_join[SIDE_STREAMS];
     /* steady-state graph of the last device-resident batch shape */
     hipGraphExec_t graph_exec;
-    uint64_t     graph_key[13];
+    uint64_t     graph_key[14];
     int          graph_valid;
     int          graph_binned;
     uint32_t     graph_launches;
@@ -337,6 +338,8 @@ static int init_buffer(myers_buffer_t *b)
     HIP_TRY(hipMalloc((void **)&b->d_results, re_b));
     HIP_TRY(hipMalloc((void **)&b->d_order, (size_t)b->max_candidates * sizeof(uint32_t)));
     HIP_TRY(hipMalloc((void **)&b->d_work, MYERS_WORK_WORDS * sizeof(uint32_t)));
+    HIP_TRY(hipMemset(b->d_work + MYERS_WORK_SPLIT, 0, MYERS_SPLIT_WORDS * sizeof(uint32_t)));
+    HIP_TRY(hipDeviceSynchronize());
     for (uint32_t i = 0; i < SIDE_STREAMS; i++) {
         HIP_TRY(hipStreamCreateWithFlags(&b->side[i], hipStreamNonBlocking));
         HIP_TRY(hipEventCreateWithFlags(&b->ev_join[i], hipEventDisableTiming));
@@ -381,6 +384,8 @@ static int create_context(myers_ctx_t **out, int device)
         if (myers_variant_occupancy_persistent(v, &occ) != 0 || occ <= 0) occ = 1;
         ctx->occupancy_p[v] = occ;
         ctx->chunk_factor[v] = 1u;
+        if (ctx->variants[v].lanes > 1u) ctx->multi_lane |= 1ull << v;
+        else if (ctx->variants[v].words >= 8u) ctx->deep |= 1ull << v;
     }
     default_bin_table(ctx);
     if (hipMalloc((void **)&ctx->d_bin_of_words, sizeof(ctx->bin_of_words)) != hipSuccess) {
@@ -653,8 +658,7 @@ static uint32_t resolve_engine(const myers_ctx_t *ctx, uint32_t flags, const bin
 static uint32_t present_by_cost(const myers_ctx_t *ctx, uint64_t present, uint32_t *out)
 {
     uint32_t n = 0;
-    for (uint32_t v = 0; v < ctx->num_variants; v++)
-        if (present & (1ull << v)) out[n++] = v;
+    for (; present; present &= present - 1u) out[n++] = (uint32_t)__builtin_ctzll(present);
     for (uint32_t i = 1; i < n; i++) {
         uint32_t x = out[i], j = i;
         while (j > 0 && ctx->variants[out[j - 1]].total_words < ctx->variants[x].total_words) {
@@ -681,7 +685,7 @@ static uint32_t present_by_cost(const myers_ctx_t *ctx, uint64_t present, uint32
  * time of the launch, max(longest chain, SIMD-time of all items / SIMDs).
  * Per column step, from single-candidate runs: one wave of W words per lane
  * ~40 + 20 W ns, a workgroup of W words per lane ~63 + 18.5 W ns.  Returns the
- * bins taken (0: none). */
+ * bins taken (0: none) and the estimated time. */
 #define LONG_ROUNDS 4u
 static double chain_ns(uint32_t max_m, uint32_t lanes, uint32_t words, int wide)
 {
@@ -690,9 +694,10 @@ static double chain_ns(uint32_t max_m, uint32_t lanes, uint32_t words, int wide)
 }
 
 static uint32_t long_plan(const myers_ctx_t *ctx, const bin_scan_t *scan, const batch_t *bt,
-                          const uint32_t *order, uint32_t n, myers_long_plan_t *lp)
+                          const uint32_t *order, uint32_t n, myers_long_plan_t *lp, double *ns)
 {
     memset(lp, 0, sizeof(*lp));
+    if (ns) *ns = 0.0;
     if (!scan->sized || bt->num_queries == 0) return 0;
     const double cpr = (double)bt->num_cands / (double)bt->num_queries;
     const double simds = (double)MYERS_LONG_WAVES * (double)ctx->num_cus;
@@ -734,6 +739,11 @@ static uint32_t long_plan(const myers_ctx_t *ctx, const bin_scan_t *scan, const 
         wide[top] = 1;
         chain[top] = c_wide;
         work = work_wide;
+    }
+    if (ns) {
+        *ns = work / simds;
+        for (uint32_t k = 0; k < nt; k++)
+            if (chain[k] > *ns) *ns = chain[k];
     }
     for (uint32_t k = 0; k < nt; k++) {            /* wide bins keep the longest-first order */
         const uint32_t v = take[k];
@@ -787,9 +797,10 @@ static slice_load_t slice_load(const myers_ctx_t *ctx, const bin_scan_t *scan, u
     slice_load_t l = {num_cands, 0.0, binned};
     if (!scan->sized || num_queries == 0) return l;
     double work = 0.0;
-    for (uint32_t v = 0; v < ctx->num_variants; v++) {
+    for (uint64_t left = scan->present & ~ctx->multi_lane; left; left &= left - 1u) {
+        const uint32_t v = (uint32_t)__builtin_ctzll(left);
         const double w = (double)ctx->variants[v].words;
-        if (ctx->variants[v].lanes == 1u) work += (double)scan->reads[v] * w * w;
+        work += (double)scan->reads[v] * w * w;
     }
     l.per_wave = work * (double)num_cands / (double)num_queries / 64.0 / (12.0 * (double)ctx->num_cus);
     return l;
@@ -848,7 +859,8 @@ static void slice_plan_add(const myers_ctx_t *ctx, myers_queue_plan_t *p, uint32
 static uint64_t wide_bins(const myers_ctx_t *ctx, const bin_scan_t *scan, const batch_t *bt)
 {
     const uint32_t engine = bt->flags & MYERS_ENGINE_MASK;
-    if (!scan->sized || scan->too_long || bt->num_queries == 0 || bt->threshold >= 0.0f ||
+    if (!(scan->present & ctx->multi_lane) || !scan->sized || scan->too_long || bt->num_queries == 0 ||
+        bt->threshold >= 0.0f ||
         (engine != MYERS_ENGINE_AUTO && engine != MYERS_ENGINE_PERSISTENT))
         return 0;
     const double cpr = (double)bt->num_cands / (double)bt->num_queries;
@@ -876,6 +888,139 @@ static uint64_t wide_bins(const myers_ctx_t *ctx, const bin_scan_t *scan, const 
     }
     const double wide = work / (double)ctx->num_cus + 0.4 * longest;
     return (wide > longest ? wide : longest) < cells / 120e3 + old_chain ? mask : 0;
+}
+
+/* Estimate of a split launch (myers_launch_split), in ns.
+ *
+ * A step of a part costs about as much as its instructions of a wave alone on
+ * its SIMD, so parts of few words shorten a candidate's chain but spend more
+ * of the chip on it, and a second wave per SIMD gains some throughput for longer
+ * chains.  Measured ns per step of a part, and of a SIMD's time per step: `kinds`.
+ * A batch takes the longer of its longest chain (every part runs about 130
+ * columns behind the one below) and the work over all SIMDs, and 0.3 of a chain
+ * more where it is more than one part per wave. */
+enum { SPLIT_KINDS = 4 };
+static const struct { uint32_t words, per_simd; double chain, work; } split_kinds[SPLIT_KINDS] = {
+    {1u, 1u, 52.0, 52.0}, {1u, 2u, 75.0, 47.0}, {2u, 1u, 70.0, 70.0}, {2u, 2u, 95.0, 59.0}};
+typedef struct {
+    double chain[SPLIT_KINDS], work[SPLIT_KINDS], items[SPLIT_KINDS];
+} split_est_t;
+
+static void split_est_add(split_est_t *e, uint32_t total_words, double m, double cands)
+{
+    for (uint32_t k = 0; k < (uint32_t)SPLIT_KINDS; k++) {
+        const uint32_t w = 64u * split_kinds[k].words;
+        const double parts = (double)((total_words + w - 1u) / w);
+        const double ns = (1.25 * m + 64.0 + 130.0 * (parts - 1.0)) * split_kinds[k].chain;
+        if (ns > e->chain[k]) e->chain[k] = ns;
+        e->items[k] += cands * parts;
+        e->work[k] += 0.9 * cands * parts * (1.25 * m + 64.0) * split_kinds[k].work;
+    }
+}
+
+static double split_est_ns(const split_est_t *e, double simds, uint32_t *best)
+{
+    double least = 0.0;
+    for (uint32_t k = 0; k < (uint32_t)SPLIT_KINDS; k++) {
+        double ns = e->work[k] / simds;
+        if (e->items[k] > simds * split_kinds[k].per_simd) ns += 0.3 * e->chain[k];
+        if (ns < e->chain[k]) ns = e->chain[k];
+        if (k == 0 || ns < least) {
+            least = ns;
+            *best = k;
+        }
+    }
+    return least;
+}
+
+/* The bins of a batch that run split over waves.  Returns the words per lane
+ * (0: none).
+ *
+ * Multi-lane bins, all of them or none: where the estimate is below that of the
+ * bit-vector launches (2-20 kb, 4 candidates each: 25-100 reads 1.6 ms against
+ * 3.0, 200 reads 2.0 against 3.5, 400 reads 3.0 against 5.6, 1,600 reads would be
+ * 11 against 8.4; one read of 20,000 bases 1.6 against 6.4; 1,100-4,000 bases:
+ * 250 reads 0.37 against 1.04, 1,000 reads 0.73 against 1.07, 2,000 reads would
+ * be 1.2 against 1.1).  One-lane bins, whose chunks of the sliced kernel take
+ * about 16.6 ns per word and step: beside multi-lane bins those of 8 words or
+ * more, most words first, while a chunk would take longer than the launch with
+ * them; without multi-lane bins all or none, which keeps the batch one launch
+ * (11 candidates per read, 1000 bases: 10 reads 121 us against 675, 300 reads 285
+ * against 680; 100-1000 bases: 100 reads 196 against 700). */
+static uint32_t split_plan(const myers_ctx_t *ctx, const bin_scan_t *scan, const batch_t *bt, const uint32_t *order,
+                           uint32_t n, myers_split_plan_t *sp, uint32_t *grid)
+{
+    const uint32_t engine = bt->flags & MYERS_ENGINE_MASK;
+    sp->n = 0;
+    *grid = 0;
+    if (!(scan->present & (ctx->multi_lane | ctx->deep)) || !scan->sized || scan->too_long || bt->num_queries == 0 ||
+        (bt->flags & MYERS_NO_LONG_LAUNCH) ||
+        (engine != MYERS_ENGINE_AUTO && engine != MYERS_ENGINE_PERSISTENT))
+        return 0;
+    const double cpr = (double)bt->num_cands / (double)bt->num_queries;
+    const double simds = 4.0 * (double)ctx->num_cus;
+    /* the binning, which a batch of one bin does without */
+    const double extra = scan->num_present == 1 ? 50e3 : 0.0;
+    split_est_t est = {{0.0}, {0.0}, {0.0}};
+    double cells = 0.0, old_chain = 0.0, old = 0.0, now = 0.0;
+    uint32_t longest = 0, best = 0, i = 0;
+    for (; i < n && ctx->variants[order[i]].lanes > 1u && sp->n < (uint32_t)MYERS_QUEUE_MAX; i++) {
+        const uint32_t v = order[i];
+        const myers_variant_desc_t *d = &ctx->variants[v];
+        if (d->lanes > 64u) return 0;
+        const double cands = scan->counted ? (double)scan->cands[v] : (double)scan->reads[v] * cpr;
+        const double m = (double)scan->max_m[v], c = chain_ns(scan->max_m[v], d->lanes, d->words, 0);
+        sp->variant[sp->n++] = v;
+        if (d->total_words > longest) longest = d->total_words;
+        if (cands <= 0.0) continue;
+        split_est_add(&est, d->total_words, m, cands);
+        cells += 0.8 * cands * 1.25 * m * m;
+        if (c > old_chain) old_chain = c;
+    }
+    if (sp->n) {
+        myers_long_plan_t lp;
+        if (scan->num_present == 1 || !long_plan(ctx, scan, bt, order, n, &lp, &old))
+            old = cells / 120e3 > old_chain ? cells / 120e3 : old_chain;
+        now = split_est_ns(&est, simds, &best);
+        if (now + extra >= old) return 0;
+    }
+    const uint32_t nlong = sp->n;
+    double slowest = 0.0;                   /* of the one-lane launch, without multi-lane bins */
+    for (; i < n && sp->n < (uint32_t)MYERS_QUEUE_MAX; i++) {
+        const uint32_t v = order[i];
+        const myers_variant_desc_t *d = &ctx->variants[v];
+        if (d->lanes > 1u || (nlong && d->words < 8u)) break;
+        const double cands = scan->counted ? (double)scan->cands[v] : (double)scan->reads[v] * cpr;
+        const double m = (double)scan->max_m[v];
+        double chunk = d->words < 8u ? 0.0 : (1.25 * m + 31.0) * (20.0 + 16.6 * (double)d->words);
+        if (cands * 1.25 * m * m / 220e3 > chunk) chunk = cands * 1.25 * m * m / 220e3;
+        if (chunk > slowest) slowest = chunk;
+        split_est_t with = est;
+        uint32_t kind = 0;
+        split_est_add(&with, d->total_words, m, cands);
+        const double then = split_est_ns(&with, simds, &kind);
+        if (nlong && then >= (now > chunk ? now : chunk)) break;
+        est = with;
+        now = then;
+        best = kind;
+        sp->variant[sp->n++] = v;
+        if (d->total_words > longest) longest = d->total_words;
+    }
+    if (!nlong && (i < n || now + extra >= slowest)) return 0;
+    /* slots for the longest window that a bin's reads can have */
+    const double cols = 32.0 * (double)longest * (1.0 + 2.0 * (double)bt->distance) + 64.0;
+    if (sp->n == 0 || !(cols >= 64.0) || cols > 1e6) return 0;
+    const uint32_t words = split_kinds[best].words;
+    for (uint32_t j = 0; j < sp->n; j++)
+        sp->parts[j] = (ctx->variants[sp->variant[j]].total_words + 64u * words - 1u) / (64u * words);
+    sp->stride = ((uint32_t)cols + 128u) / 64u * 2u + 4u;
+    sp->nslots = (uint32_t)MYERS_SPLIT_POOL_WORDS / 2u / sp->stride;
+    if (sp->nslots > (uint32_t)MYERS_SPLIT_MAX_SLOTS) sp->nslots = MYERS_SPLIT_MAX_SLOTS;
+    if (sp->nslots < (uint32_t)MYERS_SPLIT_MIN_SLOTS) return 0;
+    sp->pool = (uint64_t *)(bt->d_work + MYERS_WORK_SPLIT);
+    sp->done = bt->d_work + MYERS_WORK_SPLIT + MYERS_SPLIT_POOL_WORDS;
+    *grid = (uint32_t)ctx->num_cus * split_kinds[best].per_simd;
+    return words;
 }
 
 /* Launch one bin: variant v over a->start / count or its bin range, with a
@@ -964,7 +1109,13 @@ static int enqueue_pipeline(myers_buffer_t *b, const batch_t *bt, const bin_scan
     a.results = bt->d_results;
 
     const uint64_t wide = wide_bins(ctx, scan, bt);
-    const uint32_t engine = wide ? (uint32_t)MYERS_ENGINE_PERSISTENT : resolve_engine(ctx, bt->flags, scan, bt->num_cands);
+    uint32_t order[MYERS_MAX_VARIANTS];
+    const uint32_t n = present_by_cost(ctx, scan->present, order);
+    myers_split_plan_t sp;
+    uint32_t split_grid = 0;
+    const uint32_t split = wide ? 0u : split_plan(ctx, scan, bt, order, n, &sp, &split_grid);
+    const uint32_t engine =
+        wide || split ? (uint32_t)MYERS_ENGINE_PERSISTENT : resolve_engine(ctx, bt->flags, scan, bt->num_cands);
     b->stats.launches = 0;
     b->stats.variantsUsed = 0;
     b->binned = 0;
@@ -1027,8 +1178,6 @@ static int enqueue_pipeline(myers_buffer_t *b, const batch_t *bt, const bin_scan
     a.order = bt->d_order;
     a.bin_ranges = ranges;
     a.queue_heads = heads;
-    uint32_t order[MYERS_MAX_VARIANTS];
-    const uint32_t n = present_by_cost(ctx, scan->present, order);
     uint32_t launches = n;
     if (engine == MYERS_ENGINE_PLAIN) {
         /* one launch per length bin, in turn */
@@ -1047,13 +1196,14 @@ static int enqueue_pipeline(myers_buffer_t *b, const batch_t *bt, const bin_scan
          * others. */
         myers_long_plan_t lp;
         uint32_t nlong = 0;
-        if (wide || (bt->flags & MYERS_NO_LONG_LAUNCH)) memset(&lp, 0, sizeof(lp));
-        else nlong = long_plan(ctx, scan, bt, order, n, &lp);
+        if (wide || split || (bt->flags & MYERS_NO_LONG_LAUNCH)) memset(&lp, 0, sizeof(lp));
+        else nlong = long_plan(ctx, scan, bt, order, n, &lp, NULL);
         uint32_t rest[MYERS_MAX_VARIANTS], nrest = 0;
         for (uint32_t i = 0; i < n; i++) {
             int in_long = 0;
             for (uint32_t j = 0; j < lp.n; j++) in_long |= lp.variant[j] == order[i];
             for (uint32_t j = 0; j < lp.n_wide; j++) in_long |= lp.wide_variant[j] == order[i];
+            for (uint32_t j = 0; split && j < sp.n; j++) in_long |= sp.variant[j] == order[i];
             if (!in_long) rest[nrest++] = order[i];
         }
         myers_queue_plan_t qp[MYERS_QUEUE_CLASSES];
@@ -1066,7 +1216,7 @@ static int enqueue_pipeline(myers_buffer_t *b, const batch_t *bt, const bin_scan
             memcpy(other, rest, nrest * sizeof(uint32_t));
             nother = nrest;
         }
-        launches = (nlong ? 1u : 0u) + nqueue + nother;
+        launches = (nlong ? 1u : 0u) + (split ? 1u : 0u) + nqueue + nother;
         const int fork = launches > 1u;
         const uint32_t width = !fork ? 0u : (launches < SIDE_STREAMS ? launches : SIDE_STREAMS);
         uint32_t next = 0;    /* launches placed so far: launch k goes on side stream k % width */
@@ -1074,6 +1224,10 @@ static int enqueue_pipeline(myers_buffer_t *b, const batch_t *bt, const bin_scan
         if (fork) {
             HIP_TRY(hipEventRecord(b->ev_fork, b->stream));
             for (uint32_t j = 0; j < width; j++) HIP_TRY(hipStreamWaitEvent(b->side[j], b->ev_fork, 0));
+        }
+        if (split) {
+            rc = myers_launch_split(&a, &sp, split, split_grid, NEXT_STREAM());
+            if (rc) return hip_fail((hipError_t)rc, "split launch", __FILE__, __LINE__);
         }
         if (nlong) {
             /* successive launches start their first items a golden-ratio step
@@ -1171,17 +1325,21 @@ static int enqueue_verify(myers_buffer_t *b, const batch_t *bt, const qryInfo_t 
     memcpy(&thr_bits, &bt->threshold, sizeof(thr_bits));
     uint32_t order[MYERS_MAX_VARIANTS];
     myers_long_plan_t lp;
+    myers_split_plan_t sp;
+    uint32_t split_grid = 0;
+    const uint32_t split =
+        split_plan(b->ctx, &scan, bt, order, present_by_cost(b->ctx, scan.present, order), &sp, &split_grid);
     const uint64_t plan_key = (bt->flags & MYERS_NO_LONG_LAUNCH) ? 0u :
                               ((uint64_t)long_plan(b->ctx, &scan, bt, order,
-                                                   present_by_cost(b->ctx, scan.present, order), &lp) |
+                                                   present_by_cost(b->ctx, scan.present, order), &lp, NULL) |
                                ((uint64_t)lp.n_wide << 32));
-    const uint64_t key[13] = {(uint64_t)(uintptr_t)bt->d_peq, (uint64_t)(uintptr_t)bt->d_qinfo,
+    const uint64_t key[14] = {(uint64_t)(uintptr_t)bt->d_peq, (uint64_t)(uintptr_t)bt->d_qinfo,
                               (uint64_t)(uintptr_t)bt->d_cands, (uint64_t)(uintptr_t)bt->d_results,
                               ((uint64_t)bt->num_entries << 32) | bt->num_queries,
                               ((uint64_t)bt->num_cands << 32) | bt->flags,
                               (uint64_t)dist_bits, scan.present,
                               (uint64_t)scan.too_long, b->ctx->tune_gen, (uint64_t)thr_bits, plan_key,
-                              wide_bins(b->ctx, &scan, bt)};
+                              wide_bins(b->ctx, &scan, bt), (uint64_t)split | ((uint64_t)sp.n << 8) | ((uint64_t)split_grid << 32)};
     if (!b->graph_valid || memcmp(key, b->graph_key, sizeof(key)) != 0) {
         if (b->graph_exec) {
             hipGraphExecDestroy(b->graph_exec);

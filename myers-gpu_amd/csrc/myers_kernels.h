@@ -171,6 +171,22 @@ enum { MYERS_WIDE_SLICE_WAVES = 12 };
 uint32_t myers_wide_slice_team(uint32_t words);
 int myers_launch_wide_slice(const myers_verify_args_t *args, const myers_queue_plan_t *plan, uint32_t grid,
                             hipStream_t stream);
+/* Long reads in small batches: each candidate's rows in parts of 64 lanes x
+ * `words` (1 or 2) words, a wave each (myers_split.hip).  pool / done: the
+ * parts' hand-over, nslots slots of `stride` 64-bit words and nslots counts,
+ * zero before a launch and zero again after it. */
+enum { MYERS_SPLIT_POOL_WORDS = 3 << 20, MYERS_SPLIT_MIN_SLOTS = 64, MYERS_SPLIT_MAX_SLOTS = 8192 };
+#define MYERS_SPLIT_HEAD (MYERS_LONG_HEAD + 6u * MYERS_QUEUE_STRIDE)
+typedef struct {
+    uint32_t n;                          /* bins, in pull order */
+    uint32_t stride, nslots, reserved;
+    uint64_t *pool;
+    uint32_t *done;
+    uint32_t variant[MYERS_QUEUE_MAX];   /* variant ids (rows of bin_ranges) */
+    uint32_t parts[MYERS_QUEUE_MAX];     /* parts per candidate of each */
+} myers_split_plan_t;
+int myers_launch_split(const myers_verify_args_t *args, const myers_split_plan_t *plan, uint32_t words, uint32_t grid,
+                       hipStream_t stream);
 /* Bit planes of the packed reference (3 words per block of 32 bases, the
  * last block padded with N). */
 int myers_launch_planes(const uint32_t *ref, uint64_t ref_words, uint32_t *planes, uint32_t nblocks,
@@ -284,7 +300,9 @@ enum { MYERS_BIN_BLOCKS = 4096 };
 #define MYERS_WORK_ERR    (2u * MYERS_MAX_VARIANTS)
 #define MYERS_WORK_HEADS  (8u * MYERS_MAX_VARIANTS)
 #define MYERS_WORK_BLOCKS (MYERS_WORK_HEADS + (uint32_t)MYERS_QUEUE_WORDS)
-#define MYERS_WORK_WORDS  (MYERS_WORK_BLOCKS + (uint32_t)MYERS_BIN_WORDS)
+#define MYERS_WORK_SPLIT  (MYERS_WORK_BLOCKS + (uint32_t)MYERS_BIN_WORDS)      /* pool, then done: zero at first */
+#define MYERS_SPLIT_WORDS ((uint32_t)MYERS_SPLIT_POOL_WORDS + (uint32_t)MYERS_SPLIT_MAX_SLOTS)
+#define MYERS_WORK_WORDS  (MYERS_WORK_SPLIT + MYERS_SPLIT_WORDS)
 
 /* Static device workspace of the allocation-free entry point
  * (myersVerifyDeviceNoAlloc): a file-scope __device__ array in the kernel

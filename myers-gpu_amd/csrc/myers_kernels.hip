@@ -651,6 +651,7 @@ __global__ __launch_bounds__(64) void bin_base_kernel(uint32_t nv, uint32_t *ran
     if (threadIdx.x == 0) {
         queue_heads[MYERS_LONG_HEAD] = 0;
         queue_heads[MYERS_WIDE_HEAD] = 0;
+        queue_heads[MYERS_SPLIT_HEAD] = 0;
         for (uint32_t c = 0; c < (uint32_t)MYERS_QUEUE_CLASSES; c++) queue_heads[MYERS_QUEUE_HEAD(c)] = 0;
     }
 }
