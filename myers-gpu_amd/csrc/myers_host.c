@@ -88,6 +88,7 @@ typedef struct myers_buffer {
     resEntry_t  *h_results;
     resEntry_t  *d_results;
     uint32_t    *d_order;
+    uint32_t    *d_list;          /* threshold mode: candidates of the second launch */
     uint32_t    *d_work;          /* MYERS_WORK_WORDS: ranges | err | queue part heads | block counts */
     uint32_t    *h_err;           /* pinned copy of the binning error flag */
     hipEvent_t   ev_batch_start, ev_batch_end;
@@ -303,6 +304,7 @@ static void free_buffer(myers_buffer_t *b)
     if (b->d_cands) hipFree(b->d_cands);
     if (b->d_results) hipFree(b->d_results);
     if (b->d_order) hipFree(b->d_order);
+    if (b->d_list) hipFree(b->d_list);
     if (b->d_work) hipFree(b->d_work);
     if (b->ev_batch_start) hipEventDestroy(b->ev_batch_start);
     if (b->ev_batch_end) hipEventDestroy(b->ev_batch_end);
@@ -337,6 +339,7 @@ static int init_buffer(myers_buffer_t *b)
     HIP_TRY(hipMalloc((void **)&b->d_cands, ca_b));
     HIP_TRY(hipMalloc((void **)&b->d_results, re_b));
     HIP_TRY(hipMalloc((void **)&b->d_order, (size_t)b->max_candidates * sizeof(uint32_t)));
+    HIP_TRY(hipMalloc((void **)&b->d_list, (size_t)b->max_candidates * sizeof(uint32_t)));
     HIP_TRY(hipMalloc((void **)&b->d_work, MYERS_WORK_WORDS * sizeof(uint32_t)));
     HIP_TRY(hipMemset(b->d_work + MYERS_WORK_SPLIT, 0, MYERS_SPLIT_WORDS * sizeof(uint32_t)));
     HIP_TRY(hipDeviceSynchronize());
@@ -636,6 +639,7 @@ typedef struct {
     float       threshold;
     uint32_t   *d_work;      /* MYERS_WORK_WORDS of pipeline workspace */
     uint32_t   *d_order;     /* slot -> candidate, num_cands words */
+    uint32_t   *d_list;      /* num_cands words */
 } batch_t;
 
 /* Auto: mixed lengths go to the persistent engine.  A batch of one length bin
@@ -1086,6 +1090,14 @@ static void queue_plans(const myers_ctx_t *ctx, const uint32_t *bins, uint32_t n
     }
 }
 
+/* The variants of a plan, as a mask. */
+static uint64_t plan_bins(const myers_queue_plan_t *p)
+{
+    uint64_t bins = 0;
+    for (uint32_t i = 0; i < p->n; i++) bins |= 1ull << p->variant[i];
+    return bins;
+}
+
 /* Enqueue the whole on-device pipeline of one batch on b->stream (no timing
  * events, so that it can be captured into a graph). */
 static int enqueue_pipeline(myers_buffer_t *b, const batch_t *bt, const bin_scan_t *scan)
@@ -1217,6 +1229,10 @@ static int enqueue_pipeline(myers_buffer_t *b, const batch_t *bt, const bin_scan
             nother = nrest;
         }
         launches = (nlong ? 1u : 0u) + (split ? 1u : 0u) + nqueue + nother;
+        /* threshold mode, batches of more than a round of the one-lane kernel's
+         * waves (275K candidates of 1000 bases: 2.15 ms either way): the first
+         * rows first (slice_first_rows) */
+        const int can_filter = bt->threshold >= 0.0f && (uint64_t)bt->num_cands >= 1024u * (uint64_t)ctx->num_cus;
         const int fork = launches > 1u;
         const uint32_t width = !fork ? 0u : (launches < SIDE_STREAMS ? launches : SIDE_STREAMS);
         uint32_t next = 0;    /* launches placed so far: launch k goes on side stream k % width */
@@ -1250,8 +1266,34 @@ static int enqueue_pipeline(myers_buffer_t *b, const batch_t *bt, const bin_scan
             const int multi = c == MYERS_QUEUE_MULTI_LANE;
             const uint32_t which = !multi ? (c == MYERS_QUEUE_ONE_LANE_16 ? 2u : 3u) : (bt->threshold >= 0.0f ? 1u : 0u);
             const uint32_t grid = queue_grid(ctx, which, qp[c].ws_u4 * 16u);
-            rc = multi ? myers_launch_queue(&a, &qp[c], grid, NEXT_STREAM())
-                       : myers_launch_slice(&a, &qp[c], MYERS_SLICE_QUEUE, grid, NEXT_STREAM());
+            hipStream_t stream = NEXT_STREAM();
+            if (multi) {
+                rc = myers_launch_queue(&a, &qp[c], grid, stream);
+            } else {
+                myers_verify_args_t two = a;
+                const int filter = can_filter && c == (uint32_t)MYERS_QUEUE_ONE_LANE;
+                if (filter) {
+                    two.list = bt->d_list;
+                    two.list_ranges = bt->d_work + MYERS_WORK_LIST;
+                    two.tally = bt->d_work + MYERS_WORK_TALLY;
+                }
+                rc = myers_launch_slice(&two, &qp[c], MYERS_SLICE_QUEUE, grid, stream);
+                if (!rc && filter && group_n)
+                    rc = myers_launch_group_n(two.list_ranges, ctx->num_variants, group_n & plan_bins(&qp[c]),
+                                              bt->num_cands, two.list, bt->d_results, stream);
+                if (!rc && filter) {
+                    two.order = two.list;
+                    two.bin_ranges = two.list_ranges;
+                    two.queue_heads = heads + 1;
+                    two.list = NULL;
+                    myers_queue_plan_t rest = qp[c];
+                    rest.cls = MYERS_QUEUE_WIDE;
+                    for (uint32_t j = 0; j < rest.n; j++)
+                        rest.key[j] = myers_wide_slice_team(ctx->variants[rest.variant[j]].total_words);
+                    rc = myers_launch_wide_slice(&two, &rest, ctx->num_cus, stream);
+                    launches++;
+                }
+            }
             if (rc) return hip_fail((hipError_t)rc, "queue launch", __FILE__, __LINE__);
         }
         for (uint32_t i = 0; i < nother; i++) {
@@ -1409,7 +1451,7 @@ int myersSendEx(void *myersBuffer, float distance, uint32_t numPEQEntries, uint3
     if (numCandidates)
         SEND_TRY(hipMemcpyAsync(b->d_cands, b->h_cands, (size_t)numCandidates * sizeof(candInfo_t), hipMemcpyHostToDevice, s));
     const batch_t bt = {b->d_peq, b->d_qinfo, b->d_cands, b->d_results, numPEQEntries, numQueries,
-                        numCandidates, flags, distance, b->threshold, b->d_work, b->d_order};
+                        numCandidates, flags, distance, b->threshold, b->d_work, b->d_order, b->d_list};
     rc = enqueue_verify(b, &bt, b->h_qinfo, b->h_cands);
     if (rc) return (b->last_error = rc);
     if (numCandidates)
@@ -1528,13 +1570,13 @@ void receiveMyersBuffer(void *myersBuffer)
 static int verify_device(myers_buffer_t *b, const void *d_peq, uint32_t numPEQEntries, const void *d_qinfo,
                          uint32_t numQueries, const void *d_candidates, uint32_t numCandidates,
                          float distance, uint32_t flags, void *d_results, const qryInfo_t *h_qinfo,
-                         uint32_t *d_work, uint32_t *d_order)
+                         uint32_t *d_work, uint32_t *d_order, uint32_t *d_list)
 {
     int rc = hip_fail(hipSetDevice(b->ctx->device), "hipSetDevice", __FILE__, __LINE__);
     if (rc) return (b->last_error = rc);
     *b->h_err = 0;
     const batch_t bt = {d_peq, d_qinfo, d_candidates, d_results, numPEQEntries, numQueries, numCandidates,
-                        flags, distance, b->threshold, d_work, d_order};
+                        flags, distance, b->threshold, d_work, d_order, d_list};
     rc = enqueue_verify(b, &bt, h_qinfo, NULL);
     b->stats.cells = 0;
     b->stats.candidates = numCandidates;
@@ -1554,7 +1596,7 @@ int myersVerifyDevice(void *myersBuffer, const void *d_peq, uint32_t numPEQEntri
         return (b->last_error = MYERS_E_INVALID_ARGUMENT);
     if (numCandidates > b->max_candidates) return (b->last_error = MYERS_E_CAPACITY);
     return verify_device(b, d_peq, numPEQEntries, d_qinfo, numQueries, d_candidates, numCandidates, distance,
-                         flags, d_results, h_qinfo, b->d_work, b->d_order);
+                         flags, d_results, h_qinfo, b->d_work, b->d_order, b->d_list);
 }
 
 /* myersVerifyDevice with the pipeline workspace in the device's static
@@ -1578,7 +1620,8 @@ int myersVerifyDeviceNoAlloc(void *myersBuffer, const void *d_peq, uint32_t numP
     }
     uint32_t *scratch = b->ctx->d_scratch;
     return verify_device(b, d_peq, numPEQEntries, d_qinfo, numQueries, d_candidates, numCandidates, distance,
-                         flags, d_results, h_qinfo, scratch, scratch + MYERS_WORK_WORDS);
+                         flags, d_results, h_qinfo, scratch, scratch + MYERS_WORK_WORDS,
+                         scratch + MYERS_WORK_WORDS + MYERS_NOALLOC_MAX_CANDIDATES);
 }
 
 int myersSetThreshold(void *myersBuffer, float errorRate)

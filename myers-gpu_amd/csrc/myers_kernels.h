@@ -54,6 +54,11 @@ typedef struct {
     uint32_t        chunk_factor;  /* persistent launch: chunks per queue pull */
     void           *results;     /* resEntry_t[] in caller order */
     uint32_t       *queue_heads; /* persistent launch: MYERS_QUEUE_WORDS words of part heads */
+    /* threshold mode, one-lane queue launches, or NULL: candidates that a part
+     * of their rows does not rule out go to `list` (each bin's in the bin's own
+     * slot range, list_ranges counts them) for a second launch; tally: candidates
+     * tried so, and kept */
+    uint32_t       *list, *list_ranges, *tally;
 } myers_verify_args_t;
 
 /* Variant table compiled into the library. */
@@ -298,6 +303,8 @@ enum { MYERS_BIN_BLOCKS = 4096 };
  * order (one word per candidate) is separate. */
 #define MYERS_WORK_RANGES 0u
 #define MYERS_WORK_ERR    (2u * MYERS_MAX_VARIANTS)
+#define MYERS_WORK_LIST   (4u * MYERS_MAX_VARIANTS)     /* ranges of the second launch's lists */
+#define MYERS_WORK_TALLY  (7u * MYERS_MAX_VARIANTS)
 #define MYERS_WORK_HEADS  (8u * MYERS_MAX_VARIANTS)
 #define MYERS_WORK_BLOCKS (MYERS_WORK_HEADS + (uint32_t)MYERS_QUEUE_WORDS)
 #define MYERS_WORK_SPLIT  (MYERS_WORK_BLOCKS + (uint32_t)MYERS_BIN_WORDS)      /* pool, then done: zero at first */
@@ -312,7 +319,7 @@ enum { MYERS_BIN_BLOCKS = 4096 };
  * `device`, which must be the current device, once per device (later calls
  * return the kept address); 0 on success, else a hipError_t. */
 #define MYERS_NOALLOC_MAX_CANDIDATES (1u << 21)
-#define MYERS_SCRATCH_WORDS (MYERS_WORK_WORDS + MYERS_NOALLOC_MAX_CANDIDATES)
+#define MYERS_SCRATCH_WORDS (MYERS_WORK_WORDS + 2u * MYERS_NOALLOC_MAX_CANDIDATES)      /* workspace, order, list */
 int myers_scratch_init(int device, uint32_t **ptr);
 int myers_launch_binning(const uint32_t *qinfo, uint32_t num_queries, const void *cands, uint32_t num_cands,
                          const uint8_t *bin_of_words, uint32_t max_words, uint32_t num_variants,

@@ -637,14 +637,18 @@ __global__ __launch_bounds__(256) void bin_scan_kernel(uint32_t *block_counts, u
     if (t == 255u) ranges[2 * v + 1] = part[255];
 }
 
-// Variant ranges from the totals, and the persistent queues' part heads.
+// Variant ranges from the totals, empty lists of the second launch, and the
+// persistent queues' part heads.
 __global__ __launch_bounds__(64) void bin_base_kernel(uint32_t nv, uint32_t *ranges, uint32_t *queue_heads) {
     if (threadIdx.x == 0) {
         uint32_t acc = 0;
         for (uint32_t v = 0; v < nv; v++) {
             ranges[2 * v] = acc;
+            ranges[MYERS_WORK_LIST + 2 * v] = acc;
+            ranges[MYERS_WORK_LIST + 2 * v + 1] = 0u;
             acc += ranges[2 * v + 1];
         }
+        ranges[MYERS_WORK_TALLY] = ranges[MYERS_WORK_TALLY + 1u] = 0u;
     }
     for (uint32_t i = threadIdx.x; i < nv * (uint32_t)MYERS_QUEUE_PARTS; i += blockDim.x)
         queue_heads[i * (uint32_t)MYERS_QUEUE_STRIDE] = 0;
@@ -652,7 +656,7 @@ __global__ __launch_bounds__(64) void bin_base_kernel(uint32_t nv, uint32_t *ran
         queue_heads[MYERS_LONG_HEAD] = 0;
         queue_heads[MYERS_WIDE_HEAD] = 0;
         queue_heads[MYERS_SPLIT_HEAD] = 0;
-        for (uint32_t c = 0; c < (uint32_t)MYERS_QUEUE_CLASSES; c++) queue_heads[MYERS_QUEUE_HEAD(c)] = 0;
+        for (uint32_t c = 0; c < (uint32_t)MYERS_QUEUE_CLASSES; c++) queue_heads[MYERS_QUEUE_HEAD(c)] = queue_heads[MYERS_QUEUE_HEAD(c) + 1u] = 0;
     }
 }
 

@@ -191,6 +191,8 @@ struct SliceBatch {
     uint32_t last_block;
     float threshold;
     uint32_t nreads, max_cols;
+    // first rows only: where the candidates kept go, and the counts (list == nullptr: all rows)
+    uint32_t *list, *kept, *tally;
 };
 template <typename T>
 __device__ __forceinline__ T *uniform_ptr(T *p) {
@@ -252,6 +254,19 @@ __device__ __forceinline__ void slice_score(uint32_t hp, uint32_t hm, uint32_t c
     best = (uint32_t)end | ((uint32_t)min_score << 16);
 }
 
+// The same where only a bound from below of the least score is asked for: of
+// eight columns each, the score before them less their falls.
+__device__ __forceinline__ void slice_bound(uint32_t hp, uint32_t hm, uint32_t &best) {
+    int32_t score = (int32_t)(best & 0xFFFFu), low = (int32_t)(best >> 16);
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+        const int32_t falls = (int32_t)__builtin_popcount((hm >> (8 * q)) & 0xFFu);
+        low = min(low, score - falls);
+        score += (int32_t)__builtin_popcount((hp >> (8 * q)) & 0xFFu) - falls;
+    }
+    best = (uint32_t)score | ((uint32_t)low << 16);
+}
+
 // Planes of 32 bases of the reference.
 __device__ __forceinline__ uint3 slice_planes(const uint32_t *__restrict__ planes, uint32_t block,
                                               uint32_t last_block) {
@@ -286,7 +301,8 @@ __device__ __forceinline__ void slice_columns(const SliceBatch &a, uint4 *lds, u
 #pragma unroll
     for (int k = 0; k < kB; k++) {
         uint32_t *cd = cand + 64u * (uint32_t)k + lane;
-        const uint32_t m = cd[2 * kC];
+        uint32_t m = cd[2 * kC];
+        if (a.list != nullptr && m != ~0u) m = (uint32_t)(R * SL);      // (the word is the threshold)
         best[k] = m == ~0u ? 0u : (m | (m << 16));
         min_col[k] = php[k] = phm[k] = 0u;
         if constexpr (kCold) {
@@ -368,7 +384,8 @@ __device__ __forceinline__ void slice_columns(const SliceBatch &a, uint4 *lds, u
         // step s0 + j gave the score row's deltas of column s0 + j - (SL-1)
         const uint32_t col0 = s0 - (uint32_t)(SL - 1);              // wraps in the first block
         const uint32_t before = s0 < (uint32_t)(SL - 1) ? (uint32_t)(SL - 1) - s0 : 0u;   // steps without a column
-        bool open = a.threshold < 0.0f;                 // a candidate's result may still change
+        // a candidate's result may still change (not asked of the first rows only)
+        bool open = a.threshold < 0.0f || a.list != nullptr;
 #pragma unroll
         for (int k = 0; k < kB; k++) {
             const uint2 v = out[((uint32_t)(2 * k) + (l >> 5)) * 32u + (l & 31u)];
@@ -382,9 +399,10 @@ __device__ __forceinline__ void slice_columns(const SliceBatch &a, uint4 *lds, u
             const uint32_t seen = col0 + before, ncols = cd[kC] >> 5;
             const uint32_t left = ncols > seen ? ncols - seen : 0u;
             const uint32_t mask = (left >= 32u ? ~0u : (1u << left) - 1u) << before;
-            slice_score(transpose32(v.x, l) & mask, transpose32(v.y, l) & mask, col0, best[k], min_col[k], php[k],
-                        phm[k]);
-            if (a.threshold >= 0.0f) {
+            const uint32_t vp = transpose32(v.x, l) & mask, vm = transpose32(v.y, l) & mask;
+            if (a.list != nullptr) slice_bound(vp, vm, best[k]);
+            else slice_score(vp, vm, col0, best[k], min_col[k], php[k], phm[k]);
+            if (a.threshold >= 0.0f && a.list == nullptr) {
                 // the score falls by one per column at most: it cannot get
                 // under the threshold or the minimum so far any more where it
                 // less the columns left is not below both
@@ -403,6 +421,7 @@ __device__ __forceinline__ void slice_columns(const SliceBatch &a, uint4 *lds, u
         if (__ballot(open) == 0ull) break;
     }
     // the last columns, and the results
+    uint32_t tried = 0, kept = 0;
 #pragma unroll
     for (int k = 0; k < kB; k++) {
         const uint32_t *cd = cand + 64u * (uint32_t)k + lane;
@@ -419,6 +438,20 @@ __device__ __forceinline__ void slice_columns(const SliceBatch &a, uint4 *lds, u
         const uint32_t m = cd[2 * kC];
         const uint32_t index =
             kCold ? text[((uint32_t)(2 * k) + (lane >> 5)) * (uint32_t)S::kCols + (uint32_t)SL + (lane & 31u)].w : cd[3 * kC];
+        if (a.list != nullptr) {
+            // the first rows' least score bounds the read's from below
+            const bool keep = index != ~0u && m != ~0u && (uint32_t)min_score <= m;
+            const uint64_t keeps = __ballot(keep);
+            const uint32_t n = (uint32_t)__builtin_popcountll(keeps);
+            uint32_t at = 0;
+            if (lane == 0u && n != 0u) at = atomicAdd(a.kept, n);
+            at = (uint32_t)__builtin_amdgcn_readfirstlane((int)at);
+            if (keep) a.list[at + (uint32_t)__builtin_popcountll(keeps & ((1ull << lane) - 1ull))] = index;
+            else if (index != ~0u) a.results[index] = m == ~0u ? make_uint2(0u, kSkipScore) : make_uint2(kNoMatch, kNoMatch);
+            tried += (uint32_t)__builtin_popcountll(__ballot(index != ~0u && m != ~0u));
+            kept += n;
+            continue;
+        }
         if (index == ~0u) continue;                     // past the bin's last candidate
         uint2 r = make_uint2(0u, kSkipScore);
         if (m != ~0u) {
@@ -427,6 +460,10 @@ __device__ __forceinline__ void slice_columns(const SliceBatch &a, uint4 *lds, u
             if (a.threshold >= 0.0f && r.y > threshold_of(m, a.threshold)) r = make_uint2(kNoMatch, kNoMatch);
         }
         a.results[index] = r;
+    }
+    if (a.list != nullptr && lane == 0u) {
+        atomicAdd(a.tally, tried);
+        atomicAdd(a.tally + 1, kept);
     }
 }
 
@@ -445,6 +482,9 @@ __device__ __noinline__ bool slice_run(SliceBatch a, SliceLds *lds_at) {
     a.peq = uniform_ptr(a.peq);
     a.planes = uniform_ptr(a.planes);
     a.results = uniform_ptr(a.results);
+    a.list = uniform_ptr(a.list);
+    a.kept = uniform_ptr(a.kept);
+    a.tally = uniform_ptr(a.tally);
     a.last_block = (uint32_t)__builtin_amdgcn_readfirstlane((int)a.last_block);
     a.threshold = __uint_as_float((uint32_t)__builtin_amdgcn_readfirstlane((int)__float_as_uint(a.threshold)));
     a.max_cols = (uint32_t)__builtin_amdgcn_readfirstlane((int)a.max_cols);
@@ -565,12 +605,36 @@ __device__ __forceinline__ void slice_fallback(const myers_verify_args_t &a, uin
 #undef SLICE_FALLBACK
 }
 
-// Verify chunk `chunk` (kCands candidates) of the slot range [start, start +
-// count) of a bin whose reads have at most max_words words.  False: nothing
-// written, the chunk is one for the bit-vector kernel.
+// Threshold mode.  An alignment's first rows cost no more than all of it, so a
+// candidate whose first r rows' least score is above the threshold k of the
+// whole read has no match.  Random text scores about 0.488 r; r rows as below
+// rule out 98% of unrelated candidates (random DNA, 50-1000 bases, k of 0.05 to
+// 0.3 m): 0.23 m to 0.3 m rows for k = 0.1 m, 0.44 m to 0.52 m for k = 0.2 m.
+// The candidates kept start over with all rows, in a second launch of the
+// kernel of longer reads (32 candidates per wave, so the few chunks take half
+// as long).  Rows per lane, 0: not worth it.  11 candidates per read, one of
+// them at its place, k = 0.2 m: 50K reads of 1000 bases 3.83 -> 2.79 ms, 100K of
+// 600 bases 2.73 -> 2.43 ms; at 400 bases the work per column is most of a
+// chunk and the second launch takes what the first gains (1.56 -> 1.75 ms).
 template <int SL>
-__device__ __forceinline__ bool verify_slice(const myers_verify_args_t &a, uint32_t start, uint32_t count,
-                                             uint32_t chunk, uint32_t max_words, uint4 *lds) {
+__device__ __forceinline__ uint32_t slice_first_rows(uint32_t max_words, float threshold) {
+    const float m = 32.0f * (float)max_words;
+    const uint32_t all = 32u * max_words / (uint32_t)SL;
+    const float r = 2.05f * (float)threshold_of(32u * max_words, threshold) + 0.75f * sqrtf(m) + 6.0f;
+    const uint32_t rows = r >= m ? all : ((uint32_t)r + (uint32_t)SL) / (uint32_t)SL;
+    return SL == 32 && max_words >= 18u && 10u * rows <= 7u * all ? rows : 0u;
+}
+
+// Verify chunk `chunk` (kCands candidates) of the slot range [start, start +
+// count) of a bin whose reads have at most max_words words; of their first
+// `first` rows per lane only (0: all rows).  kSliceRefused: nothing written, the
+// chunk is one for the bit-vector kernel; kSliceShort: nothing written, some
+// read has fewer rows than `first`.
+enum SliceDone { kSliceDone, kSliceRefused, kSliceShort };
+template <int SL>
+__device__ __forceinline__ SliceDone verify_slice(const myers_verify_args_t &a, uint32_t start, uint32_t count,
+                                                  uint32_t chunk, uint32_t max_words, uint32_t first, uint32_t variant,
+                                                  uint4 *lds) {
     using S = SliceShape<SL>;
     const uint32_t lane = threadIdx.x, half = lane >> 5, ci = lane & 31u;
     const CandRec *__restrict__ cands = static_cast<const CandRec *>(a.cands);
@@ -603,10 +667,10 @@ __device__ __forceinline__ bool verify_slice(const myers_verify_args_t &a, uint3
                     if (live) {
                         // aligned window (src-api/coreMyersGPU-CC35.cu:132,144) or exact start:
                         // first text column (base 32 block + window % 32) and columns (window / 32)
-                        const uint64_t first = a.mode == 0 ? (cr.position & ~7ull) : cr.position;
+                        const uint64_t from = a.mode == 0 ? (cr.position & ~7ull) : cr.position;
                         const uint32_t ncols = a.mode == 0 ? 8u * ((n >> 3) + ((n & 7u) ? 2u : 1u)) : n;
-                        block = (uint32_t)(first >> 5);
-                        window = ((uint32_t)first & 31u) | (ncols << 5);
+                        block = (uint32_t)(from >> 5);
+                        window = ((uint32_t)from & 31u) | (ncols << 5);
                         m_hi = max(m_hi, max(m, 1u));
                         m_lo = min(m_lo, max(m, 1u));
                         cols = max(cols, ncols);
@@ -617,7 +681,7 @@ __device__ __forceinline__ bool verify_slice(const myers_verify_args_t &a, uint3
         uint32_t *cd = cand + 64 * k + lane;
         cd[0] = block;
         cd[S::kCands] = window;
-        cd[2 * S::kCands] = live ? m : ~0u;
+        cd[2 * S::kCands] = !live ? ~0u : first ? threshold_of(m, a.threshold) : m;
         cd[3 * S::kCands] = index;
         const uint32_t below = (uint32_t)__shfl_up((int)query, 1);
         const bool head = ci == 0u || below != query;
@@ -630,7 +694,7 @@ __device__ __forceinline__ bool verify_slice(const myers_verify_args_t &a, uint3
         const uint32_t n_lo = (uint32_t)__builtin_popcount((uint32_t)heads64);
         const uint32_t at = nreads + (half ? n_lo : 0u);
         // the entry and m of a run are its first candidate's: one read has one
-        if (head) tab[at + (uint32_t)__builtin_popcount(heads & upto) - 1u] = make_uint4(entry, m, run & lives, 0u);
+        if (head) tab[at + (uint32_t)__builtin_popcount(heads & upto) - 1u] = make_uint4(entry, first ? min(m, first * (uint32_t)SL) : m, run & lives, 0u);
         if (ci == 0u) first_read[(uint32_t)(2 * k) + half] = at;
         nreads += (uint32_t)__builtin_popcountll(heads64);
     }
@@ -645,17 +709,22 @@ __device__ __forceinline__ bool verify_slice(const myers_verify_args_t &a, uint3
             const uint32_t index = cand[3 * S::kCands + 64 * k + (int)lane];
             if (index != ~0u) static_cast<uint2 *>(a.results)[index] = make_uint2(0u, kSkipScore);
         }
-        return true;
+        return kSliceDone;
+    }
+    if (first) {
+        if (m_lo < first * (uint32_t)SL) return kSliceShort;
+        m_hi = m_lo = first * (uint32_t)SL;
     }
     if ((m_hi + 31u) >> 5 == (m_lo + 31u) >> 5 && max_cols < kSliceMaxCols) {
         const SliceBatch batch = {a.peq, a.planes, static_cast<uint2 *>(a.results), a.plane_blocks - 1u, a.threshold,
-                                  nreads, max_cols};
+                                  nreads, max_cols, first ? a.list + start : nullptr,
+                                  first ? a.list_ranges + 2u * variant + 1u : nullptr, first ? a.tally : nullptr};
         SliceLds *lds_at = (SliceLds *)lds;
         switch ((m_hi + (uint32_t)SL - 1u) / (uint32_t)SL) {
 #define SLICE_CASE(R)                                                                            \
     case R:                                                                                      \
         if constexpr ((R) * SL <= 32 * slice_max_words(SL))                                      \
-            return slice_run<SL, (R)>(batch, lds_at);                                            \
+            return slice_run<SL, (R)>(batch, lds_at) ? kSliceDone : kSliceRefused;               \
         break;
             SLICE_CASE(1) SLICE_CASE(2) SLICE_CASE(3) SLICE_CASE(4) SLICE_CASE(5) SLICE_CASE(6) SLICE_CASE(7)
             SLICE_CASE(8) SLICE_CASE(9) SLICE_CASE(10) SLICE_CASE(11) SLICE_CASE(12) SLICE_CASE(13) SLICE_CASE(14)
@@ -667,7 +736,7 @@ __device__ __forceinline__ bool verify_slice(const myers_verify_args_t &a, uint3
                 break;
         }
     }
-    return false;
+    return kSliceRefused;
 }
 
 }  // namespace

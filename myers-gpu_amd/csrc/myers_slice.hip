@@ -68,7 +68,22 @@ void verify_slice_kernel(myers_verify_args_t a, myers_queue_plan_t p, uint32_t m
         }
         // bins of form 1 run the bit-vector kernel (chunks of 64, as form 32)
         const uint32_t words = p.key[j] & 0xFFu;
-        if (p.key[j] >> 8 == 1u || !verify_slice<SL>(a, start, count, chunk, words, slice_lds))
+        SliceDone done = kSliceRefused;
+        if (p.key[j] >> 8 != 1u) {
+            // first rows only, while they rule out enough: of `tally`'s
+            // candidates a share below 0.75 of what the rows left out would cost
+            uint32_t first = a.list != nullptr ? slice_first_rows<SL>(words, a.threshold) : 0u;
+            if (first != 0u) {
+                const uint32_t tried = __hip_atomic_load(a.tally, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                const uint32_t kept = __hip_atomic_load(a.tally + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                const float share = 0.75f * (1.0f - (float)(first * (uint32_t)SL) / (32.0f * (float)words));
+                const bool go = tried < 16384u || (float)kept < share * (float)tried;
+                first = (uint32_t)__builtin_amdgcn_readfirstlane(go ? (int)first : 0);
+            }
+            done = verify_slice<SL>(a, start, count, chunk, words, first, p.variant[j], slice_lds);
+            if (done == kSliceShort) done = verify_slice<SL>(a, start, count, chunk, words, 0u, p.variant[j], slice_lds);
+        }
+        if (done != kSliceDone)
             slice_fallback(a, start, count, chunk, (uint32_t)SL, words, slice_lds);
     }
 }
@@ -137,6 +152,9 @@ extern "C" int myers_launch_slice(const myers_verify_args_t *args, const myers_q
     if (args == nullptr || plan == nullptr || grid == 0 || plan->n == 0 || plan->n > (uint32_t)MYERS_QUEUE_MAX || args->planes == nullptr || args->plane_blocks == 0)
         return -1;
     if (mode > (uint32_t)MYERS_SLICE_QUEUE || (mode != (uint32_t)MYERS_SLICE_QUEUE && plan->n != 1u)) return -1;
+    if (args->list != nullptr && (mode != (uint32_t)MYERS_SLICE_QUEUE || args->threshold < 0.0f ||
+                                  args->list_ranges == nullptr || args->tally == nullptr))
+        return -1;
     if (mode != (uint32_t)MYERS_SLICE_PLAIN && (args->bin_ranges == nullptr || args->queue_heads == nullptr)) return -1;
     const uint32_t lanes = plan->key[0] >> 8;
     if (plan->cls != (uint32_t)(lanes == 16u ? MYERS_QUEUE_ONE_LANE_16 : MYERS_QUEUE_ONE_LANE)) return -1;

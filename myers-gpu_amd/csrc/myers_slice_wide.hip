@@ -188,7 +188,10 @@ __device__ __forceinline__ void wide_slice_columns(const SliceBatch &a, const Wi
     const uint32_t m = cd[2 * S::kCands], index = cd[8 * S::kCands];
     if (lane >= 32u || index == ~0u) return;
     uint2 r = make_uint2(0u, kSkipScore);
-    if (m != ~0u) r = make_uint2(min_col, (uint32_t)min_score);
+    if (m != ~0u) {
+        r = make_uint2(min_col, (uint32_t)min_score);
+        if (a.threshold >= 0.0f && r.y > threshold_of(m, a.threshold)) r = make_uint2(kNoMatch, kNoMatch);
+    }
     a.results[index] = r;
 }
 
@@ -395,7 +398,7 @@ __device__ __forceinline__ bool verify_wide_slice(const myers_verify_args_t &a, 
         return true;
     }
     const SliceBatch batch = {a.peq, a.planes, static_cast<uint2 *>(a.results), a.plane_blocks - 1u, a.threshold,
-                              (uint32_t)__builtin_popcount(heads), max_cols};
+                              (uint32_t)__builtin_popcount(heads), max_cols, nullptr, nullptr, nullptr};
     SliceLds *lds_at = (SliceLds *)lds;
     const uint32_t rows = (m_hi + lanes - 1u) / lanes, lack = lanes * rows - m_lo;
     // (K rows that a lane may lack: two where the candidates are of about one
@@ -406,7 +409,7 @@ __device__ __forceinline__ bool verify_wide_slice(const myers_verify_args_t &a, 
         if (lack <= 8u * lanes) return wide_slice_run<R, 8>(batch, lds_at, waves, wave, blocks);               \
         break;
     switch (rows) {
-        WIDE_SLICE_CASE(11) WIDE_SLICE_CASE(12) WIDE_SLICE_CASE(13) WIDE_SLICE_CASE(14) WIDE_SLICE_CASE(15)
+        WIDE_SLICE_CASE(9) WIDE_SLICE_CASE(10) WIDE_SLICE_CASE(11) WIDE_SLICE_CASE(12) WIDE_SLICE_CASE(13) WIDE_SLICE_CASE(14) WIDE_SLICE_CASE(15)
         WIDE_SLICE_CASE(16) WIDE_SLICE_CASE(17) WIDE_SLICE_CASE(18) WIDE_SLICE_CASE(19) WIDE_SLICE_CASE(20)
         WIDE_SLICE_CASE(21) WIDE_SLICE_CASE(22) WIDE_SLICE_CASE(23) WIDE_SLICE_CASE(24) WIDE_SLICE_CASE(25)
         WIDE_SLICE_CASE(26) WIDE_SLICE_CASE(27) WIDE_SLICE_CASE(28) WIDE_SLICE_CASE(29) WIDE_SLICE_CASE(30)
@@ -491,7 +494,7 @@ extern "C" int myers_launch_wide_slice(const myers_verify_args_t *args, const my
                                        hipStream_t stream) {
     if (args == nullptr || plan == nullptr || grid == 0 || plan->n == 0 || plan->n > (uint32_t)MYERS_QUEUE_MAX ||
         args->planes == nullptr || args->plane_blocks == 0 || args->bin_ranges == nullptr ||
-        args->queue_heads == nullptr || args->threshold >= 0.0f || plan->cls != (uint32_t)MYERS_QUEUE_WIDE)
+        args->queue_heads == nullptr || plan->cls != (uint32_t)MYERS_QUEUE_WIDE)
         return -1;
     for (uint32_t j = 0; j < plan->n; j++) {
         myers_variant_desc_t d;
