@@ -89,8 +89,9 @@ typedef struct myers_buffer {
     resEntry_t  *d_results;
     uint32_t    *d_order;
     uint32_t    *d_list;          /* threshold mode: candidates of the second launch */
-    uint32_t    *d_work;          /* MYERS_WORK_WORDS: ranges | err | queue part heads | block counts */
-    uint32_t    *h_err;           /* pinned copy of the binning error flag */
+    uint32_t    *d_work;          /* MYERS_WORK_WORDS: ranges | queue part heads | block counts | hand-overs */
+    uint32_t    *h_err;           /* error flag of the binning, which writes it here (pinned) */
+    uint32_t    *d_err;           /* its address on the device */
     hipEvent_t   ev_batch_start, ev_batch_end;
     /* HIP events around the verification launches of each batch, in a ring
      * so that batches enqueued back to back are all timed; folded into the
@@ -334,6 +335,7 @@ static int init_buffer(myers_buffer_t *b)
     HIP_TRY(hipHostMalloc((void **)&b->h_cands, ca_b, hipHostMallocDefault));
     HIP_TRY(hipHostMalloc((void **)&b->h_results, re_b, hipHostMallocDefault));
     HIP_TRY(hipHostMalloc((void **)&b->h_err, sizeof(uint32_t), hipHostMallocDefault));
+    HIP_TRY(hipHostGetDevicePointer((void **)&b->d_err, b->h_err, 0));
     HIP_TRY(hipMalloc((void **)&b->d_peq, peq_b));
     HIP_TRY(hipMalloc((void **)&b->d_qinfo, qi_b));
     HIP_TRY(hipMalloc((void **)&b->d_cands, ca_b));
@@ -1165,10 +1167,9 @@ static int enqueue_pipeline(myers_buffer_t *b, const batch_t *bt, const bin_scan
     /* device-side binning */
     uint32_t *ranges = bt->d_work + MYERS_WORK_RANGES;
     uint32_t *heads = bt->d_work + MYERS_WORK_HEADS;
-    uint32_t *err = bt->d_work + MYERS_WORK_ERR;
     rc = myers_launch_binning((const uint32_t *)bt->d_qinfo, bt->num_queries, bt->d_cands, bt->num_cands,
                               ctx->d_bin_of_words, max_supported_words(ctx), ctx->num_variants,
-                              bt->d_work + MYERS_WORK_BLOCKS, ranges, bt->d_order, err, bt->d_results, heads,
+                              bt->d_work + MYERS_WORK_BLOCKS, ranges, bt->d_order, b->d_err, bt->d_results, heads,
                               b->stream);
     if (rc) return hip_fail((hipError_t)rc, "binning launch", __FILE__, __LINE__);
     if (group_n) {
@@ -1180,7 +1181,6 @@ static int enqueue_pipeline(myers_buffer_t *b, const batch_t *bt, const bin_scan
         rc = myers_launch_sort_len(&a, ranges, ctx->num_variants, wide, bt->num_cands, bt->d_order, b->stream);
         if (rc) return hip_fail((hipError_t)rc, "sort launch", __FILE__, __LINE__);
     }
-    HIP_TRY(hipMemcpyAsync(b->h_err, err, sizeof(uint32_t), hipMemcpyDeviceToHost, b->stream));
     if (b->mark_slot >= 0) {
         /* eager batches: the verification launches are timed apart from the binning */
         HIP_TRY(hipEventRecord(b->ev_kernel[b->mark_slot][2], b->stream));

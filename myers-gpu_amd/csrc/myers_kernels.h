@@ -302,7 +302,6 @@ enum { MYERS_BIN_BLOCKS = 4096 };
  * (128-byte aligned), then the binning block counts.  The slot -> candidate
  * order (one word per candidate) is separate. */
 #define MYERS_WORK_RANGES 0u
-#define MYERS_WORK_ERR    (2u * MYERS_MAX_VARIANTS)
 #define MYERS_WORK_LIST   (4u * MYERS_MAX_VARIANTS)     /* ranges of the second launch's lists */
 #define MYERS_WORK_TALLY  (7u * MYERS_MAX_VARIANTS)
 #define MYERS_WORK_HEADS  (8u * MYERS_MAX_VARIANTS)
@@ -313,9 +312,9 @@ enum { MYERS_BIN_BLOCKS = 4096 };
 
 /* Static device workspace of the allocation-free entry point
  * (myersVerifyDeviceNoAlloc): a file-scope __device__ array in the kernel
- * library holding MYERS_WORK_WORDS workspace words followed by the order of
- * up to MYERS_NOALLOC_MAX_CANDIDATES candidates (9.1 MB per GPU, held until
- * the process ends).  myers_scratch_init resolves its device address on
+ * library holding MYERS_WORK_WORDS workspace words followed by the order and
+ * the second launch's list of up to MYERS_NOALLOC_MAX_CANDIDATES candidates
+ * (30.5 MB per GPU, held until the process ends).  myers_scratch_init resolves its device address on
  * `device`, which must be the current device, once per device (later calls
  * return the kept address); 0 on success, else a hipError_t. */
 #define MYERS_NOALLOC_MAX_CANDIDATES (1u << 21)
@@ -323,7 +322,7 @@ enum { MYERS_BIN_BLOCKS = 4096 };
 int myers_scratch_init(int device, uint32_t **ptr);
 int myers_launch_binning(const uint32_t *qinfo, uint32_t num_queries, const void *cands, uint32_t num_cands,
                          const uint8_t *bin_of_words, uint32_t max_words, uint32_t num_variants,
-                         uint32_t *block_counts, uint32_t *ranges, uint32_t *order, uint32_t *err,
+                         uint32_t *block_counts, uint32_t *ranges, uint32_t *order, uint32_t *host_err,
                          void *results, uint32_t *queue_heads, hipStream_t stream);
 
 /* Candidates of reads with an N put together (order of the work only; the

@@ -551,10 +551,6 @@ void verify_queue_kernel(myers_verify_args_t a, myers_queue_plan_t p) {
 
 // ---------------------------------------------------------------- binning
 
-__global__ __launch_bounds__(64) void bin_reset_kernel(uint32_t *err) {
-    if (threadIdx.x == 0) *err = 0;
-}
-
 constexpr uint32_t kTooLong = 0xFFFFFFFFu;
 constexpr uint32_t kBadQuery = 0xFFFFFFFEu;
 
@@ -569,11 +565,14 @@ __device__ __forceinline__ uint32_t variant_of(const uint2 *qinfo, uint32_t num_
 // Binning is a stable partition of the candidates by variant with no global
 // atomics: block b of the count and scatter kernels owns the contiguous span
 // [b*span, (b+1)*span); bin_count writes each block's per-variant counts
-// (variant-major), bin_scan (one block per variant) turns them into each
-// block's first slot within the variant, bin_base lays the variants' ranges
-// end to end, and bin_scatter writes every candidate's
-// id at its slot in input order.  A read's candidates, adjacent in the
-// input, stay adjacent in their bin.
+// (variant-major, and behind them the errors it met), bin_scan (one block per
+// variant, one for the errors) turns them into each block's first slot within
+// the variant, and bin_scatter lays the variants' ranges end to end (every block
+// for itself; the first one writes them down) and writes every candidate's id at
+// its slot in input order.  A read's candidates, adjacent in the input, stay
+// adjacent in their bin.  Three launches: with the ranges, a reset of the error
+// word and its copy to the host as launches of their own, a binned batch took
+// 25 us longer.
 
 __device__ __forceinline__ uint32_t bin_span(uint32_t n) {
     const uint32_t span = (n + gridDim.x - 1u) / gridDim.x;
@@ -584,9 +583,9 @@ __global__ __launch_bounds__(256) void bin_count_kernel(const uint2 *qinfo, uint
                                                         const CandRec *cands,
                                                         uint32_t n, const uint8_t *bin_of_words,
                                                         uint32_t max_words, uint32_t nv,
-                                                        uint32_t *block_counts, uint32_t *err) {
-    __shared__ uint32_t hist[MYERS_MAX_VARIANTS];
-    for (uint32_t i = threadIdx.x; i < nv; i += blockDim.x) hist[i] = 0;
+                                                        uint32_t *block_counts) {
+    __shared__ uint32_t hist[MYERS_MAX_VARIANTS];      // and the errors at nv
+    for (uint32_t i = threadIdx.x; i <= nv; i += blockDim.x) hist[i] = 0;
     __syncthreads();
     const uint32_t span = bin_span(n);
     const uint32_t lo = blockIdx.x * span, hi = min(n, lo + span);
@@ -595,23 +594,35 @@ __global__ __launch_bounds__(256) void bin_count_kernel(const uint2 *qinfo, uint
         if (v < nv) {
             atomicAdd(&hist[v], 1u);
         } else {
-            atomicOr(err, v == kBadQuery ? 2u : 1u);
+            atomicOr(&hist[nv], v == kBadQuery ? 2u : 1u);
         }
     }
     __syncthreads();
-    for (uint32_t v = threadIdx.x; v < nv; v += blockDim.x) block_counts[v * gridDim.x + blockIdx.x] = hist[v];
+    for (uint32_t v = threadIdx.x; v <= nv; v += blockDim.x) block_counts[v * gridDim.x + blockIdx.x] = hist[v];
 }
 
 // One block of 256 threads per variant: an exclusive scan of the variant's
 // per-block counts (16 consecutive blocks per thread, then a scan of the 256
 // thread sums), in place, giving each count block's first slot relative to
-// the variant's range; the variant's total goes to ranges[2v+1].
+// the variant's range; the variant's total goes to ranges[2v+1].  The last
+// block joins the errors, for the host to read (host memory).
 __global__ __launch_bounds__(256) void bin_scan_kernel(uint32_t *block_counts, uint32_t nblocks,
-                                                       uint32_t *ranges) {
+                                                       uint32_t *ranges, uint32_t *host_err) {
     __shared__ uint32_t part[256];
     const uint32_t t = threadIdx.x, v = blockIdx.x;
     const uint32_t per = (nblocks + 255u) / 256u;
     uint32_t *row = block_counts + v * nblocks;
+    if (v + 1u == gridDim.x) {
+        uint32_t any = 0;
+        for (uint32_t b = t; b < nblocks; b += 256u) any |= row[b];
+        any = (__ballot(any & 1u) != 0ull ? 1u : 0u) | (__ballot(any & 2u) != 0ull ? 2u : 0u);
+        if ((t & 63u) == 0u) part[t >> 6] = any;
+        __syncthreads();
+        if (t == 0u)
+            __hip_atomic_store(host_err, part[0] | part[1] | part[2] | part[3], __ATOMIC_RELAXED,
+                               __HIP_MEMORY_SCOPE_SYSTEM);
+        return;
+    }
     uint32_t sum = 0;
     for (uint32_t k = 0; k < per; k++) {
         const uint32_t b = t * per + k;
@@ -637,29 +648,6 @@ __global__ __launch_bounds__(256) void bin_scan_kernel(uint32_t *block_counts, u
     if (t == 255u) ranges[2 * v + 1] = part[255];
 }
 
-// Variant ranges from the totals, empty lists of the second launch, and the
-// persistent queues' part heads.
-__global__ __launch_bounds__(64) void bin_base_kernel(uint32_t nv, uint32_t *ranges, uint32_t *queue_heads) {
-    if (threadIdx.x == 0) {
-        uint32_t acc = 0;
-        for (uint32_t v = 0; v < nv; v++) {
-            ranges[2 * v] = acc;
-            ranges[MYERS_WORK_LIST + 2 * v] = acc;
-            ranges[MYERS_WORK_LIST + 2 * v + 1] = 0u;
-            acc += ranges[2 * v + 1];
-        }
-        ranges[MYERS_WORK_TALLY] = ranges[MYERS_WORK_TALLY + 1u] = 0u;
-    }
-    for (uint32_t i = threadIdx.x; i < nv * (uint32_t)MYERS_QUEUE_PARTS; i += blockDim.x)
-        queue_heads[i * (uint32_t)MYERS_QUEUE_STRIDE] = 0;
-    if (threadIdx.x == 0) {
-        queue_heads[MYERS_LONG_HEAD] = 0;
-        queue_heads[MYERS_WIDE_HEAD] = 0;
-        queue_heads[MYERS_SPLIT_HEAD] = 0;
-        for (uint32_t c = 0; c < (uint32_t)MYERS_QUEUE_CLASSES; c++) queue_heads[MYERS_QUEUE_HEAD(c)] = queue_heads[MYERS_QUEUE_HEAD(c) + 1u] = 0;
-    }
-}
-
 // Write each candidate's id at its slot: per 256-candidate round, ranks within
 // a wave come from ballots, the waves' counts are added in wave order in LDS,
 // and the block's running first slot per variant advances by the round's
@@ -668,15 +656,42 @@ __global__ __launch_bounds__(256) void bin_scatter_kernel(const uint2 *qinfo, ui
                                                           const CandRec *cands,
                                                           uint32_t n, const uint8_t *bin_of_words,
                                                           uint32_t max_words, uint32_t nv,
-                                                          const uint32_t *block_first, const uint32_t *ranges,
-                                                          uint32_t *order, uint2 *results) {
+                                                          const uint32_t *block_first, uint32_t *ranges,
+                                                          uint32_t *queue_heads, uint32_t *order, uint2 *results) {
     __shared__ uint32_t next[MYERS_MAX_VARIANTS];
     __shared__ uint32_t wave_cnt[4][MYERS_MAX_VARIANTS];
     const uint32_t lane = __lane_id();
     const uint32_t wave = threadIdx.x >> 6;
     const uint64_t below = (1ull << lane) - 1ull;
-    for (uint32_t v = threadIdx.x; v < nv; v += blockDim.x)
-        next[v] = ranges[2 * v] + block_first[v * gridDim.x + blockIdx.x];
+    if (wave == 0u) {
+        // the variants' ranges from their totals (only the first block writes
+        // them, and nothing that the others read)
+        const uint32_t total = lane < nv ? ranges[2 * lane + 1] : 0u;
+        uint32_t end = total;
+        for (uint32_t o = 1; o < 64u; o <<= 1) {
+            const uint32_t y = (uint32_t)__shfl_up((int)end, o);
+            end += lane >= o ? y : 0u;
+        }
+        if (lane < nv) next[lane] = end - total + block_first[lane * gridDim.x + blockIdx.x];
+        if (blockIdx.x == 0u && lane < nv) {
+            ranges[2 * lane] = end - total;
+            // empty lists of a second launch
+            ranges[MYERS_WORK_LIST + 2 * lane] = end - total;
+            ranges[MYERS_WORK_LIST + 2 * lane + 1] = 0u;
+        }
+        if (blockIdx.x == 0u && lane < 2u) ranges[MYERS_WORK_TALLY + lane] = 0u;
+    } else if (blockIdx.x == 0u) {
+        // the queues' heads
+        const uint32_t t = threadIdx.x - 64u;
+        for (uint32_t i = t; i < nv * (uint32_t)MYERS_QUEUE_PARTS; i += 192u)
+            queue_heads[i * (uint32_t)MYERS_QUEUE_STRIDE] = 0;
+        if (t < (uint32_t)MYERS_QUEUE_PARTS) {
+            // one line each, two words used
+            queue_heads[MYERS_LONG_HEAD + t * (uint32_t)MYERS_QUEUE_STRIDE] = 0;
+            queue_heads[MYERS_LONG_HEAD + t * (uint32_t)MYERS_QUEUE_STRIDE + 1u] = 0;
+        }
+    }
+    __syncthreads();
     const uint32_t span = bin_span(n);
     const uint32_t lo = blockIdx.x * span, hi = min(n, lo + span);
     for (uint32_t r = lo; r < hi; r += 256u) {
@@ -1087,21 +1102,20 @@ extern "C" int myers_launch_binning(const uint32_t *qinfo, uint32_t num_queries,
                                     uint32_t num_cands,
                                     const uint8_t *bin_of_words, uint32_t max_words,
                                     uint32_t num_variants, uint32_t *block_counts, uint32_t *ranges,
-                                    uint32_t *order, uint32_t *err, void *results, uint32_t *queue_heads,
+                                    uint32_t *order, uint32_t *host_err, void *results, uint32_t *queue_heads,
                                     hipStream_t stream) {
-    if (num_variants == 0 || num_variants > MYERS_MAX_VARIANTS) return -1;
+    if (num_variants == 0 || num_variants >= MYERS_MAX_VARIANTS || host_err == nullptr) return -1;
     const uint2 *qi = reinterpret_cast<const uint2 *>(qinfo);
     const CandRec *cr = static_cast<const CandRec *>(cands);
     uint32_t grid = (num_cands + 1023u) / 1024u;           // about 4 rounds of 256 per block
     if (grid > (uint32_t)MYERS_BIN_BLOCKS) grid = (uint32_t)MYERS_BIN_BLOCKS;
     if (grid == 0u) grid = 1u;
-    hipLaunchKernelGGL(bin_reset_kernel, dim3(1), dim3(64), 0, stream, err);
     hipLaunchKernelGGL(bin_count_kernel, dim3(grid), dim3(256), 0, stream, qi, num_queries, cr, num_cands,
-                       bin_of_words, max_words, num_variants, block_counts, err);
-    hipLaunchKernelGGL(bin_scan_kernel, dim3(num_variants), dim3(256), 0, stream, block_counts, grid, ranges);
-    hipLaunchKernelGGL(bin_base_kernel, dim3(1), dim3(64), 0, stream, num_variants, ranges, queue_heads);
+                       bin_of_words, max_words, num_variants, block_counts);
+    hipLaunchKernelGGL(bin_scan_kernel, dim3(num_variants + 1u), dim3(256), 0, stream, block_counts, grid, ranges,
+                       host_err);
     hipLaunchKernelGGL(bin_scatter_kernel, dim3(grid), dim3(256), 0, stream, qi, num_queries, cr, num_cands,
-                       bin_of_words, max_words, num_variants, block_counts, ranges, order,
+                       bin_of_words, max_words, num_variants, block_counts, ranges, queue_heads, order,
                        static_cast<uint2 *>(results));
     return (int)hipGetLastError();
 }
