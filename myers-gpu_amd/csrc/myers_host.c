@@ -905,9 +905,10 @@ static uint64_t wide_bins(const myers_ctx_t *ctx, const bin_scan_t *scan, const 
  * A batch takes the longer of its longest chain (every part runs about 130
  * columns behind the one below) and the work over all SIMDs, and 0.3 of a chain
  * more where it is more than one part per wave. */
-enum { SPLIT_KINDS = 4 };
+enum { SPLIT_KINDS = 6 };
 static const struct { uint32_t words, per_simd; double chain, work; } split_kinds[SPLIT_KINDS] = {
-    {1u, 1u, 52.0, 52.0}, {1u, 2u, 75.0, 47.0}, {2u, 1u, 70.0, 70.0}, {2u, 2u, 95.0, 59.0}};
+    {1u, 1u, 52.0, 52.0}, {1u, 2u, 75.0, 47.0}, {2u, 1u, 70.0, 70.0}, {2u, 2u, 95.0, 59.0},
+    {4u, 1u, 105.0, 105.0}, {4u, 2u, 180.0, 85.0}};
 typedef struct {
     double chain[SPLIT_KINDS], work[SPLIT_KINDS], items[SPLIT_KINDS];
 } split_est_t;
@@ -944,8 +945,9 @@ static double split_est_ns(const split_est_t *e, double simds, uint32_t *best)
  *
  * Multi-lane bins, all of them or none: where the estimate is below that of the
  * bit-vector launches (2-20 kb, 4 candidates each: 25-100 reads 1.6 ms against
- * 3.0, 200 reads 2.0 against 3.5, 400 reads 3.0 against 5.6, 1,600 reads would be
- * 11 against 8.4; one read of 20,000 bases 1.6 against 6.4; 1,100-4,000 bases:
+ * 3.0, 200 reads 2.0 against 3.5, 400 reads 2.9 against 5.6, 800 reads 5.0
+ * against 6.3, 1,600 reads would be 9.1 against 8.4; one read of 20,000 bases 1.6
+ * against 6.4; 1,100-4,000 bases:
  * 250 reads 0.37 against 1.04, 1,000 reads 0.73 against 1.07, 2,000 reads would
  * be 1.2 against 1.1).  One-lane bins, whose chunks of the sliced kernel take
  * about 16.6 ns per word and step: beside multi-lane bins those of 8 words or
@@ -985,8 +987,9 @@ static uint32_t split_plan(const myers_ctx_t *ctx, const bin_scan_t *scan, const
     }
     if (sp->n) {
         myers_long_plan_t lp;
-        if (scan->num_present == 1 || !long_plan(ctx, scan, bt, order, n, &lp, &old))
-            old = cells / 120e3 > old_chain ? cells / 120e3 : old_chain;
+        /* (a quarter of a chain: what the tail of the long-read launch took over its estimate) */
+        if (scan->num_present > 1 && long_plan(ctx, scan, bt, order, n, &lp, &old)) old += 0.25 * old_chain;
+        else old = cells / 120e3 > old_chain ? cells / 120e3 : old_chain;
         now = split_est_ns(&est, simds, &best);
         if (now + extra >= old) return 0;
     }

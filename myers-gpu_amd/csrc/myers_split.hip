@@ -249,7 +249,7 @@ __device__ __forceinline__ void split_stage(const myers_verify_args_t &a, const 
 template <int W>
 __global__ __launch_bounds__(64 * (int)kSplitWaves) void verify_split_kernel(myers_verify_args_t a,
                                                                              myers_split_plan_t p) {
-    __shared__ SplitLds<W> split_lds[kSplitWaves];
+    __shared__ __attribute__((aligned(16))) SplitLds<W> split_lds[kSplitWaves];
     const uint32_t lane = threadIdx.x & 63u;
     SplitLds<W> &lds = split_lds[__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6))];
     uint32_t *counter = a.queue_heads + MYERS_SPLIT_HEAD;
@@ -337,7 +337,7 @@ __global__ __launch_bounds__(64 * (int)kSplitWaves) void verify_split_kernel(mye
 extern "C" int myers_launch_split(const myers_verify_args_t *args, const myers_split_plan_t *plan, uint32_t words,
                                   uint32_t grid, hipStream_t stream) {
     if (args == nullptr || plan == nullptr || grid == 0 || plan->n == 0 || plan->n > (uint32_t)MYERS_QUEUE_MAX ||
-        (words != 1u && words != 2u) || plan->pool == nullptr || plan->done == nullptr ||
+        (words != 1u && words != 2u && words != 4u) || plan->pool == nullptr || plan->done == nullptr ||
         plan->nslots < (uint32_t)MYERS_SPLIT_MIN_SLOTS || plan->nslots > (uint32_t)MYERS_SPLIT_MAX_SLOTS ||
         plan->stride == 0 || (uint64_t)plan->nslots * plan->stride * 2u > (uint64_t)MYERS_SPLIT_POOL_WORDS ||
         args->bin_ranges == nullptr || args->queue_heads == nullptr)
@@ -348,8 +348,9 @@ extern "C" int myers_launch_split(const myers_verify_args_t *args, const myers_s
             plan->parts[j] >= (uint32_t)MYERS_SPLIT_MIN_SLOTS)
             return -1;
     }
-    const void *k = words == 1u ? reinterpret_cast<const void *>(&verify_split_kernel<1>)
-                                : reinterpret_cast<const void *>(&verify_split_kernel<2>);
+    const void *k = words == 1u   ? reinterpret_cast<const void *>(&verify_split_kernel<1>)
+                    : words == 2u ? reinterpret_cast<const void *>(&verify_split_kernel<2>)
+                                  : reinterpret_cast<const void *>(&verify_split_kernel<4>);
     void *kargs[] = {const_cast<myers_verify_args_t *>(args), const_cast<myers_split_plan_t *>(plan)};
     return (int)hipLaunchKernel(k, dim3(grid), dim3(64u * kSplitWaves), kargs, 0, stream);
 }
