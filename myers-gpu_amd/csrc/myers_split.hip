@@ -27,11 +27,13 @@
 // Bound by single-wave issue: 22 to 24 VALU operations per step of one word (32
 // to 34 of two) at about 5 clocks each, 52 and 70 ns per step; the workgroup of
 // four waves and three words per lane that took such reads before needs 118 ns
-// (46 operations per word step, a barrier every 8 steps).  One candidate of
-// 20,000 bases: 6.4 ms on one wave, 2.9 on such a workgroup, 1.57 here (10
-// parts).  Blocks of 64 steps because a word's way through memory takes about
-// 2 us: with blocks of 32 steps, one ahead, the loads stalled 0.4 us per block
-// (1.98 ms).
+// (46 operations per step, a barrier every 8 steps).  Four words per lane take
+// 105 ns, or 85 ns of a SIMD's time with two waves on it: 98e12 cells per second
+// against 60e12 with two words, for batches of some hundred long reads.  One
+// candidate of 20,000 bases: 6.4 ms on one wave, 2.9 on such a workgroup, 1.57
+// here (10 parts).  Blocks of 64 steps because a word's way through memory takes
+// about 2 us: with blocks of 32 steps, one ahead, the loads stalled 0.4 us per
+// block (1.98 ms).
 #include "myers_device.h"
 
 namespace {
