@@ -990,22 +990,27 @@ static double split_est_ns(const split_est_t *e, double simds, uint32_t *best)
  * about 16.6 ns per word and step: beside multi-lane bins those of 8 words or
  * more, most words first, while a chunk would take longer than the launch with
  * them; without multi-lane bins all or none, which keeps the batch one launch
- * (11 candidates per read, 1000 bases: 10 reads 121 us against 675, 300 reads 285
- * against 680; 100-1000 bases: 100 reads 196 against 700). */
+ * (100-1000 bases, 11 candidates per read: 100 reads 129 us against 700), and
+ * where that is one bin of one part per candidate without binning (8 candidates
+ * per read: 100 reads of 100 bases 31 us against 34 with the bit-vector kernel,
+ * 200 reads would be 35.5 against 34.5; 100 reads of 250 bases 41 against 88, of
+ * 1000 bases 87 against 680, 1,000 reads of 1000 bases 415 against 680). */
 static uint32_t split_plan(const myers_ctx_t *ctx, const bin_scan_t *scan, const batch_t *bt, const uint32_t *order,
                            uint32_t n, myers_split_plan_t *sp, uint32_t *grid)
 {
     const uint32_t engine = bt->flags & MYERS_ENGINE_MASK;
     sp->n = 0;
     *grid = 0;
-    if (!(scan->present & (ctx->multi_lane | ctx->deep)) || !scan->sized || scan->too_long || bt->num_queries == 0 ||
+    if ((scan->num_present > 1 && !(scan->present & (ctx->multi_lane | ctx->deep))) || !scan->sized || scan->too_long || bt->num_queries == 0 ||
         (bt->flags & MYERS_NO_LONG_LAUNCH) ||
         (engine != MYERS_ENGINE_AUTO && engine != MYERS_ENGINE_PERSISTENT))
         return 0;
     const double cpr = (double)bt->num_cands / (double)bt->num_queries;
     const double simds = 4.0 * (double)ctx->num_cus;
-    /* the binning, which a batch of one bin does without */
-    const double extra = scan->num_present == 1 ? 50e3 : 0.0;
+    /* the binning, which a batch of one bin does without, also here if it is one
+     * part per candidate */
+    const int one = engine == MYERS_ENGINE_AUTO && scan->num_present == 1;
+    double extra = 0.0;
     split_est_t est = {{0.0}, {0.0}, {0.0}};
     double cells = 0.0, old_chain = 0.0, old = 0.0, now = 0.0;
     uint32_t longest = 0, best = 0, i = 0;
@@ -1028,6 +1033,7 @@ static uint32_t split_plan(const myers_ctx_t *ctx, const bin_scan_t *scan, const
         if (scan->num_present > 1 && long_plan(ctx, scan, bt, order, n, &lp, &old)) old += 0.25 * old_chain;
         else old = cells / 120e3 > old_chain ? cells / 120e3 : old_chain;
         now = split_est_ns(&est, simds, &best);
+        if (one && ctx->variants[sp->variant[0]].total_words > 64u * split_kinds[best].words) extra = 50e3;
         if (now + extra >= old) return 0;
     }
     const uint32_t nlong = sp->n;
@@ -1038,7 +1044,8 @@ static uint32_t split_plan(const myers_ctx_t *ctx, const bin_scan_t *scan, const
         if (d->lanes > 1u || (nlong && d->words < 8u)) break;
         const double cands = scan->counted ? (double)scan->cands[v] : (double)scan->reads[v] * cpr;
         const double m = (double)scan->max_m[v];
-        double chunk = d->words < 8u ? 0.0 : (1.25 * m + 31.0) * (20.0 + 16.6 * (double)d->words);
+        double chunk = d->words < 8u ? 1.25 * m * (40.0 + 20.0 * (double)d->words)
+                                     : (1.25 * m + 31.0) * (20.0 + 16.6 * (double)d->words);
         if (cands * 1.25 * m * m / 220e3 > chunk) chunk = cands * 1.25 * m * m / 220e3;
         if (chunk > slowest) slowest = chunk;
         split_est_t with = est;
@@ -1052,7 +1059,7 @@ static uint32_t split_plan(const myers_ctx_t *ctx, const bin_scan_t *scan, const
         sp->variant[sp->n++] = v;
         if (d->total_words > longest) longest = d->total_words;
     }
-    if (!nlong && (i < n || now + extra >= slowest)) return 0;
+    if (!nlong && (i < n || now + extra + 2e3 >= slowest)) return 0;
     /* slots for the longest window that a bin's reads can have */
     const double cols = 32.0 * (double)longest * (1.0 + 2.0 * (double)bt->distance) + 64.0;
     if (sp->n == 0 || !(cols >= 64.0) || cols > 1e6) return 0;
@@ -1188,11 +1195,15 @@ static int enqueue_pipeline(myers_buffer_t *b, const batch_t *bt, const bin_scan
     if (bt->num_cands == 0) return MYERS_SUCCESS;
     const int one_bin = engine == MYERS_ENGINE_PLAIN && scan->num_present == 1 && !scan->too_long;
     const slice_load_t load = slice_load(ctx, scan, bt->num_queries, bt->num_cands, !one_bin);
-    if (one_bin) {
+    const int one_part = split && scan->num_present == 1 && sp.parts[0] == 1u && !binned &&
+                         (bt->flags & MYERS_ENGINE_MASK) == MYERS_ENGINE_AUTO;
+    if (one_bin || one_part) {
         const uint32_t v = scan->single;
         a.start = 0;
         a.count = bt->num_cands;
-        rc = launch_bin(ctx, v, &a, &load, 0, b->stream);
+        const uint32_t waves = (bt->num_cands + 3u) / 4u;
+        rc = one_part ? myers_launch_split(&a, &sp, split, split_grid < waves ? split_grid : waves, b->stream)
+                      : launch_bin(ctx, v, &a, &load, 0, b->stream);
         if (rc) return hip_fail((hipError_t)rc, "verify launch", __FILE__, __LINE__);
         b->stats.launches = 1;
         b->stats.variantsUsed = 1;

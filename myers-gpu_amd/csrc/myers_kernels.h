@@ -179,7 +179,8 @@ int myers_launch_wide_slice(const myers_verify_args_t *args, const myers_queue_p
 /* Long reads in small batches: each candidate's rows in parts of 64 lanes x
  * `words` (1 or 2) words, a wave each (myers_split.hip).  pool / done: the
  * parts' hand-over, nslots slots of `stride` 64-bit words and nslots counts,
- * zero before a launch and zero again after it. */
+ * zero before a launch and zero again after it.  bin_ranges NULL: one bin of one
+ * part per candidate over args->start / count. */
 enum { MYERS_SPLIT_POOL_WORDS = 3 << 20, MYERS_SPLIT_MIN_SLOTS = 64, MYERS_SPLIT_MAX_SLOTS = 8192 };
 #define MYERS_SPLIT_HEAD (MYERS_LONG_HEAD + 6u * MYERS_QUEUE_STRIDE)
 typedef struct {

@@ -256,15 +256,20 @@ __global__ __launch_bounds__(64 * (int)kSplitWaves) void verify_split_kernel(mye
     SplitLds<W> &lds = split_lds[__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6))];
     uint32_t *counter = a.queue_heads + MYERS_SPLIT_HEAD;
     set_wave_prio<64>();
+    // one bin of one part per candidate needs no ranges and no counter: each wave
+    // takes every (waves of the grid)th candidate
+    const bool plain = a.bin_ranges == nullptr;
+    uint32_t next = blockIdx.x * kSplitWaves + (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     uint32_t total = 0;                                 // boundaries of the launch
-    for (uint32_t j = 0; j < p.n; j++) total += a.bin_ranges[2u * p.variant[j] + 1u] * (p.parts[j] - 1u);
+    for (uint32_t j = 0; j < p.n && !plain; j++) total += a.bin_ranges[2u * p.variant[j] + 1u] * (p.parts[j] - 1u);
     for (;;) {
-        uint32_t got = 0;
-        if (lane == 0u) got = atomicAdd(counter, 1u);
+        uint32_t got = next;
+        next += gridDim.x * kSplitWaves;
+        if (!plain && lane == 0u) got = atomicAdd(counter, 1u);
         const uint32_t item = (uint32_t)__builtin_amdgcn_readfirstlane((int)got);
-        uint32_t base = 0, bound = 0, start = 0, count = 0, parts = 1;
-        bool found = false;
-        for (uint32_t j = 0; j < p.n && !found; j++) {
+        uint32_t base = 0, bound = 0, start = a.start, count = a.count, parts = 1;
+        bool found = plain && item < count;
+        for (uint32_t j = 0; j < p.n && !found && !plain; j++) {
             start = a.bin_ranges[2u * p.variant[j]];
             count = a.bin_ranges[2u * p.variant[j] + 1u];
             parts = p.parts[j];
@@ -341,9 +346,9 @@ extern "C" int myers_launch_split(const myers_verify_args_t *args, const myers_s
     if (args == nullptr || plan == nullptr || grid == 0 || plan->n == 0 || plan->n > (uint32_t)MYERS_QUEUE_MAX ||
         (words != 1u && words != 2u && words != 4u) || plan->pool == nullptr || plan->done == nullptr ||
         plan->nslots < (uint32_t)MYERS_SPLIT_MIN_SLOTS || plan->nslots > (uint32_t)MYERS_SPLIT_MAX_SLOTS ||
-        plan->stride == 0 || (uint64_t)plan->nslots * plan->stride * 2u > (uint64_t)MYERS_SPLIT_POOL_WORDS ||
-        args->bin_ranges == nullptr || args->queue_heads == nullptr)
+        plan->stride == 0 || (uint64_t)plan->nslots * plan->stride * 2u > (uint64_t)MYERS_SPLIT_POOL_WORDS)
         return -1;
+    if (args->bin_ranges == nullptr ? plan->n != 1u || plan->parts[0] != 1u : args->queue_heads == nullptr) return -1;
     for (uint32_t j = 0; j < plan->n; j++) {
         myers_variant_desc_t d;
         if (myers_variant_desc(plan->variant[j], &d) != 0 || plan->parts[j] * 64u * words < d.total_words ||

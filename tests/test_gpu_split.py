@@ -1,4 +1,4 @@
-"""Reads of over 224 bases in small batches, their rows split over waves, against the oracle:
+"""Reads in small batches, their rows split over waves, against the oracle:
 reads of one part and of the most parts, lengths at the parts' borders, more
 hand-overs than slots, repeated launches and replayed graphs on one buffer, and
 skipped candidates between live ones."""
@@ -11,7 +11,7 @@ import oracle_lib as O
 pytestmark = pytest.mark.gpu
 
 SIZE = 2_000_000
-LENGTHS = [225, 256, 257, 700, 1023, 1024, 1025, 2047, 2048, 2049, 4096, 4097, 6145, 8192, 8193, 16385, 20000, 24575, 24576]
+LENGTHS = [97, 128, 150, 224, 225, 256, 257, 700, 1023, 1024, 1025, 2047, 2048, 2049, 4096, 4097, 6145, 8192, 8193, 16385, 20000, 24575, 24576]
 
 
 @pytest.fixture(scope="module")
