@@ -3,7 +3,7 @@
  * src-api/myers-interface.h, re-designed for one MI355X.
  *
  * Plain C over the HIP runtime C API.  Kernels are launched through the
- * extern "C" shims of myers_kernels.hip (myers_kernels.h).
+ * extern "C" shims of the .hip files (myers_kernels.h).
  *
  * Life of a batch (src-api/myersGPU.c:466-524 is the reference flow):
  *   send:    async H2D of Peq entries, qinfo and candidates on the buffer's
@@ -13,11 +13,13 @@
  *            scatter (myersGPU.c:500-513) do not exist here.
  *   launch:  the host scans qinfo (O(queries)) for the length bins present.
  *            One bin -> one launch over the candidates as they are.  More
- *            bins -> device-side binning (count, scan, base, scatter), then
- *            one launch per present bin in turn (plain engine), or one
- *            resident launch per bin on forked streams (persistent engine),
- *            where the long-read bins of a latency-bound batch share one
- *            launch (long_plan, myers_launch_long).
+ *            bins, or a large batch -> device-side binning (count, scan,
+ *            scatter), then one launch per present bin in turn (plain engine),
+ *            one queue launch per kernel class (persistent engine) or one
+ *            resident launch per bin on forked streams (binned engine).  Small
+ *            batches split their candidates over waves (split_plan), mid-sized
+ *            ones of long reads share one launch (long_plan), large ones of
+ *            long reads run the sliced kernel (wide_bins).
  *   receive: hipStreamSynchronize; results are in the pinned results buffer.
  *
  * All buffers of a library instance live on one device and share one copy
@@ -895,15 +897,16 @@ static void slice_plan_add(const myers_ctx_t *ctx, myers_queue_plan_t *p, uint32
  * are estimated, a bin's mean read counting 0.8 of its longest: a step of 12
  * waves costs 28 ns per row of a lane and 60 ns beside (T waves per chunk, steps
  * for 1.25 m columns and the lag over the waves) and the last chunks leave 0.4
- * of one chunk's time idle; the bit-vector kernels run 120e12 cells per second behind one candidate's chain.  1000-4000
- * bases, 4 candidates each: 16,000 reads 3.9 ms against 5.4 bit-vector, 8,000
- * reads 3.8 against 3.1; 2-20 kb: 20,000 reads 46 against 68, 6,400 reads 22.6
- * and 22.6, 3,200 reads 22.1 against 12.5. */
+ * of one chunk's time idle; the bit-vector kernels run 120e12 cells per second
+ * behind one candidate's chain (in threshold mode they stop unrelated
+ * candidates before the window's end).  1000-4000 bases, 4 candidates each:
+ * 16,000 reads 3.9 ms against 5.4 bit-vector, 8,000 reads 3.8 against 3.1; 2-20
+ * kb: 20,000 reads 46 against 68 (threshold mode, k of 0.2 m: 62), 6,400 reads
+ * 22.6 and 22.6, 3,200 reads 22.1 against 12.5. */
 static uint64_t wide_bins(const myers_ctx_t *ctx, const bin_scan_t *scan, const batch_t *bt)
 {
     const uint32_t engine = bt->flags & MYERS_ENGINE_MASK;
     if (!(scan->present & ctx->multi_lane) || !scan->sized || scan->too_long || bt->num_queries == 0 ||
-        bt->threshold >= 0.0f ||
         (engine != MYERS_ENGINE_AUTO && engine != MYERS_ENGINE_PERSISTENT))
         return 0;
     const double cpr = (double)bt->num_cands / (double)bt->num_queries;
@@ -930,7 +933,9 @@ static uint64_t wide_bins(const myers_ctx_t *ctx, const bin_scan_t *scan, const 
         mask |= 1ull << v;
     }
     const double wide = work / (double)ctx->num_cus + 0.4 * longest;
-    return (wide > longest ? wide : longest) < cells / 120e3 + old_chain ? mask : 0;
+    double stop = bt->threshold >= 0.0f ? 0.78 + 0.65 * (double)bt->threshold : 1.0;
+    if (stop > 1.0) stop = 1.0;
+    return (wide > longest ? wide : longest) < stop * cells / 120e3 + old_chain ? mask : 0;
 }
 
 /* Estimate of a split launch (myers_launch_split), in ns.

@@ -50,7 +50,7 @@ typedef struct {
     float           distance;
     float           threshold;   /* < 0: off; else results above (uint32)(m*threshold) get
                                     {0xFFFFFFFF, 0xFFFFFFFF}; L = 4..64 variants stop hopeless
-                                    waves */
+                                    waves, one-lane queue launches may list (below) */
     uint32_t        chunk_factor;  /* persistent launch: chunks per queue pull */
     void           *results;     /* resEntry_t[] in caller order */
     uint32_t       *queue_heads; /* persistent launch: MYERS_QUEUE_WORDS words of part heads */
@@ -167,7 +167,7 @@ uint32_t myers_slice_ws_u4(uint32_t lanes, uint32_t words);     /* LDS in 16-byt
 int myers_slice_occupancy(uint32_t lanes, uint32_t lds_bytes, int *wg_per_cu);
 int myers_launch_slice(const myers_verify_args_t *args, const myers_queue_plan_t *plan, uint32_t mode, uint32_t grid,
                        hipStream_t stream);
-/* Multi-lane variants in large batches (threshold mode off): the
+/* Multi-lane variants in large batches, and threshold mode's second launch: the
  * candidate-sliced recurrence on workgroups of MYERS_WIDE_SLICE_WAVES waves, one
  * per CU, in teams that take 32 candidates each (myers_slice_wide.hip); bins
  * ordered by myers_launch_sort_len first.  Plans of class MYERS_QUEUE_WIDE: key
@@ -298,9 +298,10 @@ enum { MYERS_BIN_BLOCKS = 4096 };
 #define MYERS_BIN_WORDS (MYERS_BIN_BLOCKS * MYERS_MAX_VARIANTS)
 
 /* Workspace of one batch's device pipeline, in u32 words: variant ranges
- * (2 per variant) and the binning error flag in the first
+ * (2 per variant), the second launch's ranges and tally in the first
  * 8 * MYERS_MAX_VARIANTS words, then the persistent queues' part heads
- * (128-byte aligned), then the binning block counts.  The slot -> candidate
+ * (128-byte aligned), then the binning block counts, then the split launch's
+ * hand-overs.  The slot -> candidate
  * order (one word per candidate) is separate. */
 #define MYERS_WORK_RANGES 0u
 #define MYERS_WORK_LIST   (4u * MYERS_MAX_VARIANTS)     /* ranges of the second launch's lists */

@@ -273,8 +273,9 @@ __device__ __forceinline__ uint3 slice_planes(const uint32_t *__restrict__ plane
     return *reinterpret_cast<const uint3 *>(planes + (size_t)min(block, last_block) * 3u);
 }
 
-// The columns of a chunk whose read planes are in place (kN: SliceN).  A lane's candidates: number 64 k + lane of the chunk, i.e. candidate lane % 32
-// of group 2 k + lane / 32.
+// The columns of a chunk whose read planes are in place (kN: SliceN).  A lane's
+// candidates: number 64 k + lane of the chunk, i.e. candidate lane % 32 of group
+// 2 k + lane / 32.
 template <int SL, int R, int kN>
 __device__ __forceinline__ void slice_columns(const SliceBatch &a, uint4 *lds, uint32_t lane, const uint32_t (&r0)[R],
                                               const uint32_t (&r1)[R], const uint32_t (&rn)[kN == kRowsN ? R : 1],
@@ -468,7 +469,8 @@ __device__ __forceinline__ void slice_columns(const SliceBatch &a, uint4 *lds, u
 }
 
 // A chunk whose live candidates' reads all have W words and at most R SL
-// bases; tab: its `nreads` distinct reads in chunk order, {entry, m, live candidates of the group, 0}.
+// bases; tab: its `nreads` distinct reads in chunk order, {entry, m, live
+// candidates of the group, 0}.
 // False (nothing written) if a read's Peq is not one code per base.
 //
 // Not inlined: as a part of one large kernel, the register allocator spills

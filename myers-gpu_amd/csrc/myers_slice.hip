@@ -4,9 +4,9 @@
 
 namespace {
 
-// One kernel per form (SL lanes per group) for every engine.  It is compiled for three waves per
-// SIMD (168 VGPRs): 32 rows per lane take 128, and three waves issue the
-// double-rate operations at 0.41 per clock against 0.35 with two.
+// One kernel per form (SL lanes per group) for every engine.  It is compiled for
+// three waves per SIMD (168 VGPRs): 32 rows per lane take 128, and three waves
+// issue the double-rate operations at 0.41 per clock against 0.35 with two.
 //   MYERS_SLICE_PLAIN  one bin, a fixed grid strides over its chunks
 //   MYERS_SLICE_RANGES one bin, a resident grid pulls guided ranges of chunks
 //   MYERS_SLICE_QUEUE  every bin of the plan, one chunk at a time from a
@@ -149,7 +149,8 @@ extern "C" int myers_slice_occupancy(uint32_t lanes, uint32_t lds_bytes, int *wg
 
 extern "C" int myers_launch_slice(const myers_verify_args_t *args, const myers_queue_plan_t *plan, uint32_t mode,
                                   uint32_t grid, hipStream_t stream) {
-    if (args == nullptr || plan == nullptr || grid == 0 || plan->n == 0 || plan->n > (uint32_t)MYERS_QUEUE_MAX || args->planes == nullptr || args->plane_blocks == 0)
+    if (args == nullptr || plan == nullptr || grid == 0 || plan->n == 0 || plan->n > (uint32_t)MYERS_QUEUE_MAX ||
+        args->planes == nullptr || args->plane_blocks == 0)
         return -1;
     if (mode > (uint32_t)MYERS_SLICE_QUEUE || (mode != (uint32_t)MYERS_SLICE_QUEUE && plan->n != 1u)) return -1;
     if (args->list != nullptr && (mode != (uint32_t)MYERS_SLICE_QUEUE || args->threshold < 0.0f ||

@@ -24,12 +24,16 @@ def library():
         yield ref, m
 
 
-def check(ref, m, b, mode, flags=0):
+def check(ref, m, b, mode, flags=0, threshold=-1.0):
     want = O.myers_batch(ref, SIZE, b["peq"], b["qinfo"], b["cands"], 0.1, mode)
     # twice the bit-vector kernels' time for one chunk's longest
     size = int(b["qinfo"][:, 1].max())
     times = 1 + int(2 * 120e12 * (1.25 * size + 1200) * 1e-6 / (1.25 * float(size) ** 2) / len(b["cands"]))
+    if threshold >= 0:
+        want = O.apply_threshold(b["qinfo"], b["cands"], want, threshold)
+    m.set_threshold(threshold)
     got = m.verify(b["peq"], b["qinfo"], np.tile(b["cands"], times), 0.1, flags=mode | flags)
+    m.set_threshold(-1.0)
     np.testing.assert_array_equal(got.reshape(times, -1, 2), np.broadcast_to(want, (times,) + want.shape))
 
 
@@ -50,6 +54,7 @@ def test_ragged_lengths(library, lo, hi):
     b = M.synth_batch(M.make_spec(lo, 45, log_uniform=(lo, hi), err_range=(0.0, 0.12), candidates=3, distance=0.1), ref,
                       SIZE)
     check(ref, m, b, M.WINDOW_ALIGNED)
+    check(ref, m, b, M.WINDOW_EXACT, threshold=0.08)
 
 
 @pytest.mark.parametrize("length", [1500, 5000, 7000, 9000])
