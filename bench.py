@@ -53,16 +53,17 @@ CUS, CLOCK_HZ = 256, 2.4e9
 PEAK_VALU_OPS = CUS * 128 * CLOCK_HZ
 PEAK_SINGLE_ISSUE_OPS = CUS * 64 * CLOCK_HZ                 # one instruction per quad-cycle
 PEAK_HBM_GBS = 8000.0
-# Algorithmic VALU ops per 32 cells (one u32 word of one column):
-#   K_GFX950 = 10: and, add-with-carry, 3 three-input logic ops (Xh, Ph, Pv),
-#   Mh and, Mv and, Xv or, 2 funnel shifts -- the recurrence's minimum on gfx950.
-#   7 of them issue at the double rate, the carry add and the two funnel
-#   shifts at the single rate: 6.5 single-issue slots per word, which caps
-#   this op mix at 10/6.5 x PEAK_SINGLE_ISSUE_OPS = 60.5e12 ops/s (194 TCUPS).
+# Algorithmic VALU ops per 32 cells (one row of one column for 32 candidates):
+#   K_GFX950 = 7: the match bit (two three-input logic ops), D0, and the four
+#   output deltas (two ands, two three-input ops) -- the cell recurrence's
+#   minimum on gfx950, all of them double rate, so the op mix can reach the
+#   dual-issue peak (359 TCUPS nominal; 245 at the issue rate of three waves
+#   per SIMD).  The bit-vector form (32 rows of one candidate per word) needs
+#   10: 7 double-rate and 3 single-rate ones.
 #   K_REF = 18: the reference's u32 formulation (src/myers-4bits.c:117-134).
-K_GFX950 = 10
+K_GFX950 = 7
 K_REF = 18
-OP_MIX_SLOTS = 7 * 0.5 + 3 * 1.0
+OP_MIX_SLOTS = 7 * 0.5
 PEAK_OP_MIX_OPS = PEAK_SINGLE_ISSUE_OPS * K_GFX950 / OP_MIX_SLOTS
 
 CONFIGS = {
@@ -412,8 +413,8 @@ def measure_serving(m, ref, ref_size, loads, seconds, batch_cells=0, engine=0, s
 
 
 def roofline(cells, kernel_ms, hbm_bytes, traffic, kernel):
-    """VALU roofline of one launch: algorithmic ops (K_GFX950 per word-column
-    of the nominal cells) over the verification launches' HIP-event time."""
+    """VALU roofline of one launch: algorithmic ops (K_GFX950 per 32 of
+    the nominal cells) over the verification launches' HIP-event time."""
     kernel_s = kernel_ms / 1e3
     achieved = cells * K_GFX950 / 32.0 / kernel_s
     hbm = hbm_bytes / kernel_s / 1e9
@@ -431,7 +432,7 @@ def roofline(cells, kernel_ms, hbm_bytes, traffic, kernel):
         "peak_note": "256 CUs x 128 lane-ops/clk x 2.4 GHz: the dual-issue VALU rate",
         "op_mix_ceiling": {"peak": PEAK_OP_MIX_OPS / 1e12, "unit": "TOP/s", "frac": achieved / PEAK_OP_MIX_OPS,
                            "gcups": PEAK_OP_MIX_OPS / (K_GFX950 / 32.0) / 1e9,
-                           "note": "7 double-rate + 3 single-rate ops per word: 6.5 single-issue slots"},
+                           "note": "7 double-rate ops per 32 cells: 3.5 single-issue slots"},
         "ratio_to_single_issue_peak": achieved / PEAK_SINGLE_ISSUE_OPS,
         "ratio_reference_ops_to_peak": cells * K_REF / 32.0 / kernel_s / PEAK_VALU_OPS,
         "hbm": {"achieved": hbm, "peak": PEAK_HBM_GBS, "unit": "GB/s", "frac": hbm / PEAK_HBM_GBS,

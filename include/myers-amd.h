@@ -46,8 +46,8 @@ typedef enum {
 #define MYERS_WINDOW_EXACT     1u  /* exact start: n columns from the position
                                       (src/myers-4bits.c:100-147) */
 /* Engine selection (extension).  AUTO: the plain engine for a batch of one
- * length bin of up to 2048 candidates per CU, the persistent engine
- * otherwise. */
+ * length bin of up to 2048 candidates per CU (small ones with each candidate's
+ * rows split over lanes and waves), the persistent engine otherwise. */
 #define MYERS_ENGINE_AUTO       0u
 #define MYERS_ENGINE_PLAIN      (1u << 4)  /* one launch per length bin */
 #define MYERS_ENGINE_PERSISTENT (2u << 4)  /* one persistent launch over a length-binned device queue
@@ -57,9 +57,9 @@ typedef enum {
 /* Capture the batch's on-device pipeline (binning + kernels) into a HIP
  * graph once per batch shape and replay it (extension). */
 #define MYERS_USE_GRAPH         (1u << 6)
-/* Persistent engine: do not give the long-read bins of a small batch their
- * own latency-ordered launch; every bin goes into the queue launches
- * (extension; throughput scheduling only). */
+/* Persistent engine: do not give the bins of a small batch a launch ordered for
+ * latency (long reads together, or candidates split over waves); every bin goes
+ * into the queue launches (extension; scheduling only). */
 #define MYERS_NO_LONG_LAUNCH    (1u << 7)
 
 /* Longest query supported, in bases (extension: the reference stops at 4096,
@@ -126,14 +126,11 @@ int myersReceiveEx(void *myersBuffer);
  * minimum score is <= (uint32)((float)m * errorRate) exactly as without the
  * threshold, and every other verified candidate as
  * {column 0xFFFFFFFF, score 0xFFFFFFFF}; skipped candidates keep
- * {0, 0xFFFFFFFF}.  Kernels for queries of up to 1024 bases then skip the
- * rows whose distance already exceeds the threshold (Ukkonen cut-off), and
- * the multi-lane kernels of per-bin launches stop a wave once none of its
- * candidates can get under the threshold.  In binned batches a probe of each
- * such query's first 32 bases orders those candidates so that the ones
- * likely under the threshold share waves (the order of the work only; the
- * results stay in the caller's order).  errorRate < 0 switches the mode off
- * (the default). */
+ * {0, 0xFFFFFFFF}.  Large batches of queries of 545 to 1024 bases then run
+ * the first rows of every candidate and all rows of those only that these do
+ * not rule out, and the multi-lane kernels of queue and per-bin launches stop
+ * a wave once none of its candidates can get under the threshold.
+ * errorRate < 0 switches the mode off (the default). */
 #define MYERS_NO_MATCH 0xFFFFFFFFu
 int   myersSetThreshold(void *myersBuffer, float errorRate);
 float myersGetThreshold(void *myersBuffer);
