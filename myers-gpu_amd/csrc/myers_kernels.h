@@ -220,10 +220,12 @@ int myers_launch_planes(const uint32_t *ref, uint64_t ref_words, uint32_t *plane
  *   finish:  the wave adds its item's candidates to the request's device
  *            counter; the wave that completes the request writes the
  *            request's ticket to flags[slot] after its results are visible.
- *   exit:    every wave leaves when *host_stop equals the launch's `gen` and
- *            no item is left, or after idle_ticks (its own s_memrealtime
- *            ticks, 100 MHz) in which no ring's head moved; so every launch
- *            ends by itself.
+ *   exit:    every wave leaves when *host_stop equals the launch's `gen`, or
+ *            after idle_ticks (its own s_memrealtime ticks, 100 MHz) in which
+ *            no ring's head moved; so every launch ends by itself.  The first
+ *            wave to leave closes the launch for all (dev[MYERS_SERVE_STOP] =
+ *            gen): the others finish the item they hold and take no more, and
+ *            items left in the rings are the next launch's.
  * Item and request counters are u32 and compared modulo 2^32. */
 typedef struct {
     uint32_t key;          /* lanes << 8 | words of the chunk's variant */

@@ -68,9 +68,15 @@ __device__ __forceinline__ bool serve_take(uint32_t *head, uint32_t *dtail, uint
 // Lane 0: the next item's index in its ring (`ring`), or false when the wave
 // must exit.  A long item is taken only with the SIMD's count below
 // long_per_simd; the caller lowers it when the item is done.  The wave
-// leaves when the host's stop generation is seen, or after idle_ticks in
-// which no item of either ring was claimed anywhere (the rings' heads did
-// not move), measured on this wave's own real-time counter.  An idle wave
+// leaves when the stop generation is seen, or after idle_ticks in which no
+// item of either ring was claimed anywhere (the rings' heads did not move),
+// measured on this wave's own real-time counter; it then sets the stop
+// generation itself, so that the whole grid leaves with it.  Leaving one by
+// one thins the launch: a wave that ends a long item after the last claim
+// starts its idle time later than the rest, and requests that arrive once the
+// rest has left keep those few waves busy, so that the launch neither ends
+// nor gets its grid back (seen under load after pauses of ~50 ms: 1-5e6
+// candidates/s where the full grid serves 10.5e6).  An idle wave
 // backs off from ~3 us to ~220 us between polls, so that a grid of idle
 // waves does not flood the memory system with atomics while a few waves run
 // long chains; its count of polls without progress bounds the wait as well
@@ -82,6 +88,7 @@ __device__ bool serve_claim(const myers_serve_args_t &s, uint32_t simd, uint32_t
     uint32_t idle = 0, polls = 0, heads = 0xFFFFFFFFu;
     uint64_t t_idle = __builtin_amdgcn_s_memrealtime();
     for (;;) {
+        if (__hip_atomic_load(dstop, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == s.gen) return false;
         // a long item, if fewer than long_per_simd long items run on this SIMD
         uint32_t *hl = s.dev + MYERS_SERVE_HEAD, *tl = s.dev + MYERS_SERVE_DTAIL;
         uint32_t running = __hip_atomic_load(busy, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -139,8 +146,10 @@ __device__ bool serve_claim(const myers_serve_args_t &s, uint32_t simd, uint32_t
                 continue;
             }
         }
-        if (__hip_atomic_load(dstop, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == s.gen) return false;
-        if (now - t_idle > s.idle_ticks || polls > (1u << 17)) return false;
+        if (now - t_idle > s.idle_ticks || polls > (1u << 17)) {
+            __hip_atomic_store(dstop, s.gen, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            return false;
+        }
         idle = idle < 64u ? idle + 1u : 64u;
         for (uint32_t k = 0; k < idle; k++) __builtin_amdgcn_s_sleep(127);
     }

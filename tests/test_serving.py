@@ -113,6 +113,25 @@ def test_resident_window_modes_and_threshold(mode):
         m.set_threshold(-1.0)
 
 
+def test_resident_pauses_around_the_idle_exit():
+    """Bursts after pauses on both sides of the idle time (50 ms): the grid may
+    be leaving, with its last waves on long reads, when a burst arrives.  Each
+    burst's items are done by that launch or the next."""
+    announce("resident server, pauses around the idle exit")
+    ref, reqs = make_pool(47)
+    want = [oracle_req(ref, r) for r in reqs]
+    with M.Myers(ref, REF_SIZE, num_buffers=1, avg_query=800, cands_per_query=11, buffer_bytes=256 << 20) as m:
+        with M.Server(m, distance=0.1, flags=M.SERVE_RESIDENT) as sv:
+            for pause_ms in [40, 48, 50, 51, 52, 55, 60, 75, 0]:
+                made = [M.Server.request(*r) for r in reqs]
+                for t in [sv.submit(x[0]) for x in made]:
+                    sv.wait(t)
+                done = time.perf_counter()
+                for (req, keep), w in zip(made, want):
+                    np.testing.assert_array_equal(keep[3], w, err_msg=f"before pause {pause_ms} ms")
+                time.sleep(max(0.0, pause_ms / 1e3 - (time.perf_counter() - done)))
+
+
 @pytest.mark.parametrize("serve", MODES, ids=MODE_IDS)
 def test_open_loop_poisson(serve):
     announce(f"serve open loop flags={serve}")
