@@ -255,7 +255,8 @@ __device__ __forceinline__ void slice_score(uint32_t hp, uint32_t hm, uint32_t c
 }
 
 // The same where only a bound from below of the least score is asked for: of
-// eight columns each, the score before them less their falls.
+// eight columns each, the score before them less their falls (which can be
+// below zero where rises lie between them, a score cannot).
 __device__ __forceinline__ void slice_bound(uint32_t hp, uint32_t hm, uint32_t &best) {
     int32_t score = (int32_t)(best & 0xFFFFu), low = (int32_t)(best >> 16);
 #pragma unroll
@@ -264,7 +265,7 @@ __device__ __forceinline__ void slice_bound(uint32_t hp, uint32_t hm, uint32_t &
         low = min(low, score - falls);
         score += (int32_t)__builtin_popcount((hp >> (8 * q)) & 0xFFu) - falls;
     }
-    best = (uint32_t)score | ((uint32_t)low << 16);
+    best = (uint32_t)score | ((uint32_t)max(low, 0) << 16);
 }
 
 // Planes of 32 bases of the reference.
