@@ -1236,8 +1236,10 @@ static int enqueue_pipeline(myers_buffer_t *b, const batch_t *bt, const bin_scan
     uint32_t *ranges = bt->d_work + MYERS_WORK_RANGES;
     uint32_t *heads = bt->d_work + MYERS_WORK_HEADS;
     if (group_n || wide) {
+        /* (up to the longest read that a bin holds: a size near 2^32 counts as one of
+         * no words in the binning, and its Peq is not there) */
         rc = myers_launch_read_n(&a, bt->num_cands, group_n ? 32u * GROUP_N_WORDS : 32u * myers_slice_max_words(32u),
-                                 wide ? ~0u : 32u * myers_slice_max_words(32u), b->stream);
+                                 32u * (wide ? max_supported_words(ctx) : myers_slice_max_words(32u)), b->stream);
         if (rc) return hip_fail((hipError_t)rc, "read N launch", __FILE__, __LINE__);
     }
     if (group_n) {
