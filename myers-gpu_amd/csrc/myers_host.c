@@ -93,7 +93,8 @@ typedef struct myers_buffer {
     void        *hd_peq, *hd_qinfo, *hd_cands, *hd_results;     /* the host arrays' addresses on the device */
     uint32_t    *d_order;
     uint32_t    *d_list;          /* threshold mode: candidates of the second launch */
-    uint32_t    *d_work;          /* MYERS_WORK_WORDS: ranges | queue part heads | block counts | hand-overs */
+    uint32_t    *d_work;          /* MYERS_WORK_WORDS: ranges | queue part heads | block counts */
+    uint32_t    *d_split;         /* the split launch's pool */
     uint32_t    *h_err;           /* error flag of the binning, which writes it here (pinned) */
     uint32_t    *d_err;           /* its address on the device */
     hipEvent_t   ev_batch_start, ev_batch_end;
@@ -121,6 +122,7 @@ typedef struct myers_buffer {
     int          binned;
     uint32_t     num_candidates;
     myersStats_t stats;
+    myers_launch_info_t ran, graph_ran;
 } myers_buffer_t;
 
 static void load_default_tuning(myers_ctx_t *ctx);
@@ -311,6 +313,7 @@ static void free_buffer(myers_buffer_t *b)
     if (b->d_order) hipFree(b->d_order);
     if (b->d_list) hipFree(b->d_list);
     if (b->d_work) hipFree(b->d_work);
+    if (b->d_split) hipFree(b->d_split);
     if (b->ev_batch_start) hipEventDestroy(b->ev_batch_start);
     if (b->ev_batch_end) hipEventDestroy(b->ev_batch_end);
     for (uint32_t i = 0; i < EV_RING; i++) {
@@ -351,7 +354,8 @@ static int init_buffer(myers_buffer_t *b)
     HIP_TRY(hipMalloc((void **)&b->d_order, (size_t)b->max_candidates * sizeof(uint32_t)));
     HIP_TRY(hipMalloc((void **)&b->d_list, (size_t)b->max_candidates * sizeof(uint32_t)));
     HIP_TRY(hipMalloc((void **)&b->d_work, MYERS_WORK_WORDS * sizeof(uint32_t)));
-    HIP_TRY(hipMemset(b->d_work + MYERS_WORK_SPLIT, 0, MYERS_SPLIT_WORDS * sizeof(uint32_t)));
+    HIP_TRY(hipMalloc((void **)&b->d_split, MYERS_SPLIT_WORDS * sizeof(uint32_t)));
+    HIP_TRY(hipMemset(b->d_split, 0, MYERS_SPLIT_WORDS * sizeof(uint32_t)));
     HIP_TRY(hipDeviceSynchronize());
     for (uint32_t i = 0; i < SIDE_STREAMS; i++) {
         HIP_TRY(hipStreamCreateWithFlags(&b->side[i], hipStreamNonBlocking));
@@ -683,6 +687,7 @@ typedef struct {
     uint32_t   *d_work;      /* MYERS_WORK_WORDS of pipeline workspace */
     uint32_t   *d_order;     /* slot -> candidate, num_cands words */
     uint32_t   *d_list;      /* num_cands words */
+    uint32_t   *d_split;     /* the split launch's pool, or NULL */
 } batch_t;
 
 static int large_batch(const myers_ctx_t *ctx, uint32_t num_cands)
@@ -1075,14 +1080,16 @@ static uint32_t split_plan(const myers_ctx_t *ctx, const bin_scan_t *scan, const
     const double cols = 32.0 * (double)longest * (1.0 + 2.0 * (double)bt->distance) + 64.0;
     if (sp->n == 0 || !(cols >= 64.0) || cols > 1e6) return 0;
     const uint32_t words = split_kinds[best].words;
-    for (uint32_t j = 0; j < sp->n; j++)
+    for (uint32_t j = 0; j < sp->n; j++) {
         sp->parts[j] = (ctx->variants[sp->variant[j]].total_words + 64u * words - 1u) / (64u * words);
+        if (sp->parts[j] > 1u && bt->d_split == NULL) return 0;
+    }
     sp->stride = ((uint32_t)cols + 128u) / 64u * 2u + 4u;
     sp->nslots = (uint32_t)MYERS_SPLIT_POOL_WORDS / 2u / sp->stride;
     if (sp->nslots > (uint32_t)MYERS_SPLIT_MAX_SLOTS) sp->nslots = MYERS_SPLIT_MAX_SLOTS;
     if (sp->nslots < (uint32_t)MYERS_SPLIT_MIN_SLOTS) return 0;
-    sp->pool = (uint64_t *)(bt->d_work + MYERS_WORK_SPLIT);
-    sp->done = bt->d_work + MYERS_WORK_SPLIT + MYERS_SPLIT_POOL_WORDS;
+    sp->pool = (uint64_t *)bt->d_split;
+    sp->done = bt->d_split ? bt->d_split + MYERS_SPLIT_POOL_WORDS : NULL;
     *grid = (uint32_t)ctx->num_cus * split_kinds[best].per_simd;
     return words;
 }
@@ -1202,6 +1209,7 @@ static int enqueue_pipeline(myers_buffer_t *b, const batch_t *bt, const bin_scan
     b->stats.launches = 0;
     b->stats.variantsUsed = 0;
     b->binned = 0;
+    memset(&b->ran, 0, sizeof(b->ran));
     int rc;
     if (bt->num_cands == 0) return MYERS_SUCCESS;
     const int one_bin = engine == MYERS_ENGINE_PLAIN && scan->num_present == 1 && !scan->too_long;
@@ -1216,6 +1224,8 @@ static int enqueue_pipeline(myers_buffer_t *b, const batch_t *bt, const bin_scan
         rc = one_part ? myers_launch_split(&a, &sp, split, split_grid < waves ? split_grid : waves, b->stream)
                       : launch_bin(ctx, v, &a, &load, 0, b->stream);
         if (rc) return hip_fail((hipError_t)rc, "verify launch", __FILE__, __LINE__);
+        b->ran.ran = one_part ? MYERS_RAN_SPLIT : MYERS_RAN_BIN;
+        b->ran.split_words = one_part ? split : 0u;
         b->stats.launches = 1;
         b->stats.variantsUsed = 1;
         return MYERS_SUCCESS;
@@ -1266,6 +1276,7 @@ static int enqueue_pipeline(myers_buffer_t *b, const batch_t *bt, const bin_scan
         for (uint32_t i = 0; i < n; i++) {
             rc = launch_bin(ctx, order[i], &a, &load, 0, b->stream);
             if (rc) return hip_fail((hipError_t)rc, "verify launch", __FILE__, __LINE__);
+            b->ran.ran |= MYERS_RAN_BIN;
         }
     } else {
         /* Persistent engines.  The long-read bins of a latency-bound batch
@@ -1314,6 +1325,11 @@ static int enqueue_pipeline(myers_buffer_t *b, const batch_t *bt, const bin_scan
         if (split) {
             rc = myers_launch_split(&a, &sp, split, split_grid, NEXT_STREAM());
             if (rc) return hip_fail((hipError_t)rc, "split launch", __FILE__, __LINE__);
+            b->ran.ran |= MYERS_RAN_SPLIT;
+            for (uint32_t j = 0; j < sp.n; j++)
+                if (sp.parts[j] > 1u) b->ran.ran |= MYERS_RAN_HANDOVERS;
+            b->ran.split_words = split;
+            b->ran.split_slots = sp.nslots;
         }
         if (nlong) {
             /* successive launches start their first items a golden-ratio step
@@ -1323,6 +1339,7 @@ static int enqueue_pipeline(myers_buffer_t *b, const batch_t *bt, const bin_scan
             lp.rotate = wg * MYERS_LONG_WAVES;
             rc = myers_launch_long(&a, &lp, ctx->num_cus, NEXT_STREAM());
             if (rc) return hip_fail((hipError_t)rc, "long-read launch", __FILE__, __LINE__);
+            b->ran.ran |= MYERS_RAN_LONG;
         }
         /* (longest reads first) */
         for (uint32_t k = 0; k < (uint32_t)MYERS_QUEUE_CLASSES; k++) {
@@ -1331,9 +1348,11 @@ static int enqueue_pipeline(myers_buffer_t *b, const batch_t *bt, const bin_scan
             if (c == MYERS_QUEUE_WIDE) {
                 rc = myers_launch_wide_slice(&a, &qp[c], ctx->num_cus, NEXT_STREAM());
                 if (rc) return hip_fail((hipError_t)rc, "queue launch", __FILE__, __LINE__);
+                b->ran.ran |= MYERS_RAN_WIDE_SLICE;
                 continue;
             }
             const int multi = c == MYERS_QUEUE_MULTI_LANE;
+            b->ran.ran |= multi ? MYERS_RAN_QUEUE : MYERS_RAN_SLICE;
             const uint32_t which = !multi ? (c == MYERS_QUEUE_ONE_LANE_16 ? 2u : 3u) : (bt->threshold >= 0.0f ? 1u : 0u);
             const uint32_t grid = queue_grid(ctx, which, qp[c].ws_u4 * 16u);
             hipStream_t stream = NEXT_STREAM();
@@ -1361,6 +1380,7 @@ static int enqueue_pipeline(myers_buffer_t *b, const batch_t *bt, const bin_scan
                     for (uint32_t j = 0; j < rest.n; j++)
                         rest.key[j] = myers_wide_slice_team(ctx->variants[rest.variant[j]].total_words);
                     rc = myers_launch_wide_slice(&two, &rest, ctx->num_cus, stream);
+                    b->ran.ran |= MYERS_RAN_FIRST_ROWS;
                     launches++;
                 }
             }
@@ -1369,6 +1389,7 @@ static int enqueue_pipeline(myers_buffer_t *b, const batch_t *bt, const bin_scan
         for (uint32_t i = 0; i < nother; i++) {
             rc = launch_bin(ctx, other[i], &a, &load, 1, NEXT_STREAM());
             if (rc) return hip_fail((hipError_t)rc, "persistent launch", __FILE__, __LINE__);
+            b->ran.ran |= MYERS_RAN_BIN;
         }
 #undef NEXT_STREAM
         for (uint32_t j = 0; j < width; j++) {
@@ -1480,11 +1501,13 @@ static int enqueue_verify(myers_buffer_t *b, const batch_t *bt, const qryInfo_t 
         b->graph_valid = 1;
         b->graph_binned = b->binned;
         b->graph_launches = b->stats.launches;
+        b->graph_ran = b->ran;
         b->stats.graphCaptures++;
     }
     if ((rc = timing_begin(b, &slot))) return rc;
     HIP_TRY(hipGraphLaunch(b->graph_exec, b->stream));
     b->binned = b->graph_binned;
+    b->ran = b->graph_ran;
     b->stats.launches = b->graph_launches;
     b->stats.variantsUsed = b->graph_launches;
     return timing_end(b, slot, b->graph_launches);
@@ -1552,7 +1575,8 @@ int myersSendEx(void *myersBuffer, float distance, uint32_t numPEQEntries, uint3
         SEND_TRY(hipMemcpyAsync(b->d_cands, b->h_cands, (size_t)numCandidates * sizeof(candInfo_t), hipMemcpyHostToDevice, s));
     const batch_t bt = {direct ? b->hd_peq : (void *)b->d_peq, direct ? b->hd_qinfo : (void *)b->d_qinfo,
                         direct ? b->hd_cands : (void *)b->d_cands, direct ? b->hd_results : (void *)b->d_results,
-                        numPEQEntries, numQueries, numCandidates, flags, distance, b->threshold, b->d_work, b->d_order, b->d_list};
+                        numPEQEntries, numQueries, numCandidates, flags, distance, b->threshold, b->d_work, b->d_order, b->d_list,
+                        b->d_split};
     rc = enqueue_verify(b, &bt, b->h_qinfo, b->h_cands);
     if (rc) return (b->last_error = rc);
     if (numCandidates && !direct)
@@ -1582,6 +1606,14 @@ static int finish_batch(myers_buffer_t *b, int with_batch_events)
     b->stats.binned = (uint32_t)b->binned;
     if (b->binned && (*b->h_err & 1u)) return MYERS_E_QUERY_TOO_LONG;
     if (b->binned && (*b->h_err & 2u)) return MYERS_E_INVALID_ARGUMENT;
+    return MYERS_SUCCESS;
+}
+
+int myers_launch_info(void *myersBuffer, myers_launch_info_t *out)
+{
+    const myers_buffer_t *b = (const myers_buffer_t *)myersBuffer;
+    if (b == NULL || out == NULL) return MYERS_E_INVALID_ARGUMENT;
+    *out = b->ran;
     return MYERS_SUCCESS;
 }
 
@@ -1671,13 +1703,13 @@ void receiveMyersBuffer(void *myersBuffer)
 static int verify_device(myers_buffer_t *b, const void *d_peq, uint32_t numPEQEntries, const void *d_qinfo,
                          uint32_t numQueries, const void *d_candidates, uint32_t numCandidates,
                          float distance, uint32_t flags, void *d_results, const qryInfo_t *h_qinfo,
-                         uint32_t *d_work, uint32_t *d_order, uint32_t *d_list)
+                         uint32_t *d_work, uint32_t *d_order, uint32_t *d_list, uint32_t *d_split)
 {
     int rc = hip_fail(hipSetDevice(b->ctx->device), "hipSetDevice", __FILE__, __LINE__);
     if (rc) return (b->last_error = rc);
     *b->h_err = 0;
     const batch_t bt = {d_peq, d_qinfo, d_candidates, d_results, numPEQEntries, numQueries, numCandidates,
-                        flags, distance, b->threshold, d_work, d_order, d_list};
+                        flags, distance, b->threshold, d_work, d_order, d_list, d_split};
     rc = enqueue_verify(b, &bt, h_qinfo, NULL);
     b->stats.cells = 0;
     b->stats.candidates = numCandidates;
@@ -1697,13 +1729,15 @@ int myersVerifyDevice(void *myersBuffer, const void *d_peq, uint32_t numPEQEntri
         return (b->last_error = MYERS_E_INVALID_ARGUMENT);
     if (numCandidates > b->max_candidates) return (b->last_error = MYERS_E_CAPACITY);
     return verify_device(b, d_peq, numPEQEntries, d_qinfo, numQueries, d_candidates, numCandidates, distance,
-                         flags, d_results, h_qinfo, b->d_work, b->d_order, b->d_list);
+                         flags, d_results, h_qinfo, b->d_work, b->d_order, b->d_list, b->d_split);
 }
 
 /* myersVerifyDevice with the pipeline workspace in the device's static
  * array instead of the buffer's: nothing is allocated.  Every call on one
- * GPU shares that array (the binning kernels re-initialise the parts that
- * must start at zero), so calls that overlap on one GPU race. */
+ * GPU shares that array, so calls that overlap on one GPU race; the binning
+ * kernels re-initialise every part that must start at zero, so such calls
+ * spoil no later one.  The split launch's pool does not start anew (and its
+ * waves wait for each other), so no candidate runs in several parts here. */
 int myersVerifyDeviceNoAlloc(void *myersBuffer, const void *d_peq, uint32_t numPEQEntries, const void *d_qinfo,
                              uint32_t numQueries, const void *d_candidates, uint32_t numCandidates,
                              float distance, uint32_t flags, void *d_results, const qryInfo_t *h_qinfo)
@@ -1722,7 +1756,7 @@ int myersVerifyDeviceNoAlloc(void *myersBuffer, const void *d_peq, uint32_t numP
     uint32_t *scratch = b->ctx->d_scratch;
     return verify_device(b, d_peq, numPEQEntries, d_qinfo, numQueries, d_candidates, numCandidates, distance,
                          flags, d_results, h_qinfo, scratch, scratch + MYERS_WORK_WORDS,
-                         scratch + MYERS_WORK_WORDS + MYERS_NOALLOC_MAX_CANDIDATES);
+                         scratch + MYERS_WORK_WORDS + MYERS_NOALLOC_MAX_CANDIDATES, NULL);
 }
 
 int myersSetThreshold(void *myersBuffer, float errorRate)

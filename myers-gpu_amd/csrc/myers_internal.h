@@ -11,6 +11,21 @@
  * work is pending, negative on a HIP error. */
 int myers_buffer_ready(void *myersBuffer);
 
+/* The launches of a buffer's last batch, for tests of the dispatch: MYERS_RAN_*
+ * bits, and the split launch's words per lane and slots (0 without one). */
+enum { MYERS_RAN_BIN = 1,            /* a launch per bin */
+       MYERS_RAN_SLICE = 2,          /* sliced kernel, reads up to 1024 bases */
+       MYERS_RAN_FIRST_ROWS = 4,     /* their first rows, and the rest of those kept */
+       MYERS_RAN_WIDE_SLICE = 8,     /* sliced kernel of longer reads */
+       MYERS_RAN_QUEUE = 16,         /* multi-lane queue launch */
+       MYERS_RAN_LONG = 32,          /* long-read launch */
+       MYERS_RAN_SPLIT = 64,         /* split launch */
+       MYERS_RAN_HANDOVERS = 128 };  /* ... of several parts per candidate */
+typedef struct {
+    uint32_t ran, split_words, split_slots;
+} myers_launch_info_t;
+int myers_launch_info(void *myersBuffer, myers_launch_info_t *out);
+
 /* What the resident server needs from a library instance: the device, the
  * resident reference, the buffer's threshold, and for every read length in
  * words the variant the resident kernel runs it with (the bin table's

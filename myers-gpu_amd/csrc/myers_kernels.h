@@ -177,11 +177,15 @@ uint32_t myers_wide_slice_team(uint32_t words);
 int myers_launch_wide_slice(const myers_verify_args_t *args, const myers_queue_plan_t *plan, uint32_t grid,
                             hipStream_t stream);
 /* Long reads in small batches: each candidate's rows in parts of 64 lanes x
- * `words` (1 or 2) words, a wave each (myers_split.hip).  pool / done: the
+ * `words` (1, 2 or 4) words, a wave each (myers_split.hip).  pool / done: the
  * parts' hand-over, nslots slots of `stride` 64-bit words and nslots counts,
- * zero before a launch and zero again after it.  bin_ranges NULL: one bin of one
+ * zero before a launch and zero again after it (NULL: one part per candidate in
+ * every bin).  A wave waits without end for words that another launch's waves
+ * take or leave behind, so launches that can overlap never share a pool: each
+ * buffer has its own, on its own stream.  bin_ranges NULL: one bin of one
  * part per candidate over args->start / count. */
 enum { MYERS_SPLIT_POOL_WORDS = 3 << 20, MYERS_SPLIT_MIN_SLOTS = 64, MYERS_SPLIT_MAX_SLOTS = 8192 };
+#define MYERS_SPLIT_WORDS ((uint32_t)MYERS_SPLIT_POOL_WORDS + (uint32_t)MYERS_SPLIT_MAX_SLOTS)     /* pool, then done */
 #define MYERS_SPLIT_HEAD (MYERS_LONG_HEAD + 6u * MYERS_QUEUE_STRIDE)
 typedef struct {
     uint32_t n;                          /* bins, in pull order */
@@ -302,23 +306,20 @@ enum { MYERS_BIN_BLOCKS = 4096 };
 /* Workspace of one batch's device pipeline, in u32 words: variant ranges
  * (2 per variant), the second launch's ranges and tally in the first
  * 8 * MYERS_MAX_VARIANTS words, then the persistent queues' part heads
- * (128-byte aligned), then the binning block counts, then the split launch's
- * hand-overs.  The slot -> candidate
- * order (one word per candidate) is separate. */
+ * (128-byte aligned), then the binning block counts.  The slot -> candidate
+ * order (one word per candidate) and the split launch's pool are separate. */
 #define MYERS_WORK_RANGES 0u
 #define MYERS_WORK_LIST   (4u * MYERS_MAX_VARIANTS)     /* ranges of the second launch's lists */
 #define MYERS_WORK_TALLY  (7u * MYERS_MAX_VARIANTS)
 #define MYERS_WORK_HEADS  (8u * MYERS_MAX_VARIANTS)
 #define MYERS_WORK_BLOCKS (MYERS_WORK_HEADS + (uint32_t)MYERS_QUEUE_WORDS)
-#define MYERS_WORK_SPLIT  (MYERS_WORK_BLOCKS + (uint32_t)MYERS_BIN_WORDS)      /* pool, then done: zero at first */
-#define MYERS_SPLIT_WORDS ((uint32_t)MYERS_SPLIT_POOL_WORDS + (uint32_t)MYERS_SPLIT_MAX_SLOTS)
-#define MYERS_WORK_WORDS  (MYERS_WORK_SPLIT + MYERS_SPLIT_WORDS)
+#define MYERS_WORK_WORDS  (MYERS_WORK_BLOCKS + (uint32_t)MYERS_BIN_WORDS)
 
 /* Static device workspace of the allocation-free entry point
  * (myersVerifyDeviceNoAlloc): a file-scope __device__ array in the kernel
  * library holding MYERS_WORK_WORDS workspace words followed by the order and
  * the second launch's list of up to MYERS_NOALLOC_MAX_CANDIDATES candidates
- * (30.5 MB per GPU, held until the process ends).  myers_scratch_init resolves its device address on
+ * (17.9 MB per GPU, held until the process ends).  myers_scratch_init resolves its device address on
  * `device`, which must be the current device, once per device (later calls
  * return the kept address); 0 on success, else a hipError_t. */
 #define MYERS_NOALLOC_MAX_CANDIDATES (1u << 21)

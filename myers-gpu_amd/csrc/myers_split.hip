@@ -344,7 +344,7 @@ __global__ __launch_bounds__(64 * (int)kSplitWaves) void verify_split_kernel(mye
 extern "C" int myers_launch_split(const myers_verify_args_t *args, const myers_split_plan_t *plan, uint32_t words,
                                   uint32_t grid, hipStream_t stream) {
     if (args == nullptr || plan == nullptr || grid == 0 || plan->n == 0 || plan->n > (uint32_t)MYERS_QUEUE_MAX ||
-        (words != 1u && words != 2u && words != 4u) || plan->pool == nullptr || plan->done == nullptr ||
+        (words != 1u && words != 2u && words != 4u) || (plan->pool == nullptr) != (plan->done == nullptr) ||
         plan->nslots < (uint32_t)MYERS_SPLIT_MIN_SLOTS || plan->nslots > (uint32_t)MYERS_SPLIT_MAX_SLOTS ||
         plan->stride == 0 || (uint64_t)plan->nslots * plan->stride * 2u > (uint64_t)MYERS_SPLIT_POOL_WORDS)
         return -1;
@@ -352,7 +352,7 @@ extern "C" int myers_launch_split(const myers_verify_args_t *args, const myers_s
     for (uint32_t j = 0; j < plan->n; j++) {
         myers_variant_desc_t d;
         if (myers_variant_desc(plan->variant[j], &d) != 0 || plan->parts[j] * 64u * words < d.total_words ||
-            plan->parts[j] >= (uint32_t)MYERS_SPLIT_MIN_SLOTS)
+            plan->parts[j] >= (uint32_t)MYERS_SPLIT_MIN_SLOTS || (plan->parts[j] > 1u && plan->pool == nullptr))
             return -1;
     }
     const void *k = words == 1u   ? reinterpret_cast<const void *>(&verify_split_kernel<1>)
