@@ -73,7 +73,9 @@ typedef struct {
                                    as the reference does (src-api/myersGPU.c:24-47) */
     uint32_t reserved;
     uint64_t bufferBytes;       /* device bytes per buffer used to size capacities;
-                                   0 = min(95% of free HBM / numBuffers, 2 GiB) */
+                                   0 = min(95% of free HBM / numBuffers, 2 GiB).  Beside
+                                   them a buffer takes 1.1 MB, and 12.6 MB more from its first
+                                   small batch of long reads on (not on a full device) */
 } myersConfig_t;
 
 /* Timing and counters of a buffer's last batch (extension). */

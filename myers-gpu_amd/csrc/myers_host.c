@@ -92,9 +92,8 @@ typedef struct myers_buffer {
     resEntry_t  *d_results;
     void        *hd_peq, *hd_qinfo, *hd_cands, *hd_results;     /* the host arrays' addresses on the device */
     uint32_t    *d_order;
-    uint32_t    *d_list;          /* threshold mode: candidates of the second launch */
     uint32_t    *d_work;          /* MYERS_WORK_WORDS: ranges | queue part heads | block counts */
-    uint32_t    *d_split;         /* the split launch's pool */
+    uint32_t    *d_split;         /* the split launch's pool, from its first use on (split_pool) */
     uint32_t    *h_err;           /* error flag of the binning, which writes it here (pinned) */
     uint32_t    *d_err;           /* its address on the device */
     hipEvent_t   ev_batch_start, ev_batch_end;
@@ -311,7 +310,6 @@ static void free_buffer(myers_buffer_t *b)
     if (b->d_cands) hipFree(b->d_cands);
     if (b->d_results) hipFree(b->d_results);
     if (b->d_order) hipFree(b->d_order);
-    if (b->d_list) hipFree(b->d_list);
     if (b->d_work) hipFree(b->d_work);
     if (b->d_split) hipFree(b->d_split);
     if (b->ev_batch_start) hipEventDestroy(b->ev_batch_start);
@@ -352,11 +350,7 @@ static int init_buffer(myers_buffer_t *b)
     HIP_TRY(hipMalloc((void **)&b->d_cands, ca_b));
     HIP_TRY(hipMalloc((void **)&b->d_results, re_b));
     HIP_TRY(hipMalloc((void **)&b->d_order, (size_t)b->max_candidates * sizeof(uint32_t)));
-    HIP_TRY(hipMalloc((void **)&b->d_list, (size_t)b->max_candidates * sizeof(uint32_t)));
     HIP_TRY(hipMalloc((void **)&b->d_work, MYERS_WORK_WORDS * sizeof(uint32_t)));
-    HIP_TRY(hipMalloc((void **)&b->d_split, MYERS_SPLIT_WORDS * sizeof(uint32_t)));
-    HIP_TRY(hipMemset(b->d_split, 0, MYERS_SPLIT_WORDS * sizeof(uint32_t)));
-    HIP_TRY(hipDeviceSynchronize());
     for (uint32_t i = 0; i < SIDE_STREAMS; i++) {
         HIP_TRY(hipStreamCreateWithFlags(&b->side[i], hipStreamNonBlocking));
         HIP_TRY(hipEventCreateWithFlags(&b->ev_join[i], hipEventDisableTiming));
@@ -686,8 +680,8 @@ typedef struct {
     float       threshold;
     uint32_t   *d_work;      /* MYERS_WORK_WORDS of pipeline workspace */
     uint32_t   *d_order;     /* slot -> candidate, num_cands words */
-    uint32_t   *d_list;      /* num_cands words */
-    uint32_t   *d_split;     /* the split launch's pool, or NULL */
+    uint32_t   *d_list;      /* num_cands words, or NULL */
+    myers_buffer_t *pool_of; /* the buffer whose pool the split launch may use, or NULL */
 } batch_t;
 
 static int large_batch(const myers_ctx_t *ctx, uint32_t num_cands)
@@ -993,6 +987,33 @@ static double split_est_ns(const split_est_t *e, double simds, uint32_t *best)
     return least;
 }
 
+/* The split launch's pool of a buffer, allocated (12.6 MB, 0.3 ms) and zeroed when a
+ * batch of the buffer first needs it, so that a buffer takes no more memory than
+ * its batches use.  NULL (and another launch) if there is no room, or a caller
+ * captures the stream. */
+static uint32_t *split_pool(myers_buffer_t *b)
+{
+    if (b == NULL || b->d_split) return b ? b->d_split : NULL;
+    hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(b->stream, &capture) != hipSuccess || capture != hipStreamCaptureStatusNone) return NULL;
+    /* (relaxed: the allocation does not end another thread's capture) */
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    if (hipThreadExchangeStreamCaptureMode(&mode) != hipSuccess) return NULL;
+    void *pool = NULL;
+    const hipError_t e = hipMalloc(&pool, MYERS_SPLIT_WORDS * sizeof(uint32_t));
+    (void)hipThreadExchangeStreamCaptureMode(&mode);
+    if (e != hipSuccess) {
+        (void)hipGetLastError();
+        return NULL;
+    }
+    if (hip_fail(hipMemsetAsync(pool, 0, MYERS_SPLIT_WORDS * sizeof(uint32_t), b->stream), "hipMemsetAsync", __FILE__,
+                 __LINE__)) {
+        hipFree(pool);
+        return NULL;
+    }
+    return b->d_split = (uint32_t *)pool;
+}
+
 /* The bins of a batch that run split over waves.  Returns the words per lane
  * (0: none).
  *
@@ -1080,16 +1101,17 @@ static uint32_t split_plan(const myers_ctx_t *ctx, const bin_scan_t *scan, const
     const double cols = 32.0 * (double)longest * (1.0 + 2.0 * (double)bt->distance) + 64.0;
     if (sp->n == 0 || !(cols >= 64.0) || cols > 1e6) return 0;
     const uint32_t words = split_kinds[best].words;
+    uint32_t *pool = NULL;
     for (uint32_t j = 0; j < sp->n; j++) {
         sp->parts[j] = (ctx->variants[sp->variant[j]].total_words + 64u * words - 1u) / (64u * words);
-        if (sp->parts[j] > 1u && bt->d_split == NULL) return 0;
+        if (sp->parts[j] > 1u && pool == NULL && (pool = split_pool(bt->pool_of)) == NULL) return 0;
     }
     sp->stride = ((uint32_t)cols + 128u) / 64u * 2u + 4u;
     sp->nslots = (uint32_t)MYERS_SPLIT_POOL_WORDS / 2u / sp->stride;
     if (sp->nslots > (uint32_t)MYERS_SPLIT_MAX_SLOTS) sp->nslots = MYERS_SPLIT_MAX_SLOTS;
     if (sp->nslots < (uint32_t)MYERS_SPLIT_MIN_SLOTS) return 0;
-    sp->pool = (uint64_t *)bt->d_split;
-    sp->done = bt->d_split ? bt->d_split + MYERS_SPLIT_POOL_WORDS : NULL;
+    sp->pool = (uint64_t *)pool;
+    sp->done = pool ? pool + MYERS_SPLIT_POOL_WORDS : NULL;
     *grid = (uint32_t)ctx->num_cus * split_kinds[best].per_simd;
     return words;
 }
@@ -1313,7 +1335,7 @@ static int enqueue_pipeline(myers_buffer_t *b, const batch_t *bt, const bin_scan
         /* threshold mode, batches of more than a round of the one-lane kernel's
          * waves (275K candidates of 1000 bases: 2.15 ms either way): the first
          * rows first (slice_first_rows) */
-        const int can_filter = bt->threshold >= 0.0f && (uint64_t)bt->num_cands >= 1024u * (uint64_t)ctx->num_cus;
+        const int can_filter = bt->threshold >= 0.0f && bt->d_list && (uint64_t)bt->num_cands >= 1024u * (uint64_t)ctx->num_cus;
         const int fork = launches > 1u;
         const uint32_t width = !fork ? 0u : (launches < SIDE_STREAMS ? launches : SIDE_STREAMS);
         uint32_t next = 0;    /* launches placed so far: launch k goes on side stream k % width */
@@ -1547,6 +1569,17 @@ static int reads_host_arrays(const myers_buffer_t *b, uint32_t flags, uint32_t n
     return b->ctx->variants[bin[first]].lanes == 1u;
 }
 
+/* Room for the second launch's list (threshold mode) of a batch in the buffer's
+ * arrays: what its candidates or Peq entries leave free, else NULL (every row of
+ * every candidate then runs at once). */
+static uint32_t *spare_list(const myers_buffer_t *b, uint32_t entries, uint32_t cands)
+{
+    const uint64_t need = (uint64_t)cands * sizeof(uint32_t);
+    if ((uint64_t)(b->max_candidates - cands) * sizeof(candInfo_t) >= need) return (uint32_t *)(b->d_cands + cands);
+    if ((uint64_t)(b->max_peq_entries - entries) * sizeof(qryEntry_t) >= need) return (uint32_t *)(b->d_peq + entries);
+    return NULL;
+}
+
 int myersSendEx(void *myersBuffer, float distance, uint32_t numPEQEntries, uint32_t numQueries,
                 uint32_t numCandidates, uint32_t flags)
 {
@@ -1575,8 +1608,8 @@ int myersSendEx(void *myersBuffer, float distance, uint32_t numPEQEntries, uint3
         SEND_TRY(hipMemcpyAsync(b->d_cands, b->h_cands, (size_t)numCandidates * sizeof(candInfo_t), hipMemcpyHostToDevice, s));
     const batch_t bt = {direct ? b->hd_peq : (void *)b->d_peq, direct ? b->hd_qinfo : (void *)b->d_qinfo,
                         direct ? b->hd_cands : (void *)b->d_cands, direct ? b->hd_results : (void *)b->d_results,
-                        numPEQEntries, numQueries, numCandidates, flags, distance, b->threshold, b->d_work, b->d_order, b->d_list,
-                        b->d_split};
+                        numPEQEntries, numQueries, numCandidates, flags, distance, b->threshold, b->d_work, b->d_order,
+                        spare_list(b, numPEQEntries, numCandidates), b};
     rc = enqueue_verify(b, &bt, b->h_qinfo, b->h_cands);
     if (rc) return (b->last_error = rc);
     if (numCandidates && !direct)
@@ -1703,13 +1736,13 @@ void receiveMyersBuffer(void *myersBuffer)
 static int verify_device(myers_buffer_t *b, const void *d_peq, uint32_t numPEQEntries, const void *d_qinfo,
                          uint32_t numQueries, const void *d_candidates, uint32_t numCandidates,
                          float distance, uint32_t flags, void *d_results, const qryInfo_t *h_qinfo,
-                         uint32_t *d_work, uint32_t *d_order, uint32_t *d_list, uint32_t *d_split)
+                         uint32_t *d_work, uint32_t *d_order, uint32_t *d_list, myers_buffer_t *pool_of)
 {
     int rc = hip_fail(hipSetDevice(b->ctx->device), "hipSetDevice", __FILE__, __LINE__);
     if (rc) return (b->last_error = rc);
     *b->h_err = 0;
     const batch_t bt = {d_peq, d_qinfo, d_candidates, d_results, numPEQEntries, numQueries, numCandidates,
-                        flags, distance, b->threshold, d_work, d_order, d_list, d_split};
+                        flags, distance, b->threshold, d_work, d_order, d_list, pool_of};
     rc = enqueue_verify(b, &bt, h_qinfo, NULL);
     b->stats.cells = 0;
     b->stats.candidates = numCandidates;
@@ -1728,8 +1761,9 @@ int myersVerifyDevice(void *myersBuffer, const void *d_peq, uint32_t numPEQEntri
         (numCandidates && (!d_peq || !d_qinfo || !d_candidates || !d_results)))
         return (b->last_error = MYERS_E_INVALID_ARGUMENT);
     if (numCandidates > b->max_candidates) return (b->last_error = MYERS_E_CAPACITY);
+    /* (the buffer's own candidate array is free meanwhile: the second launch's list) */
     return verify_device(b, d_peq, numPEQEntries, d_qinfo, numQueries, d_candidates, numCandidates, distance,
-                         flags, d_results, h_qinfo, b->d_work, b->d_order, b->d_list, b->d_split);
+                         flags, d_results, h_qinfo, b->d_work, b->d_order, (uint32_t *)b->d_cands, b);
 }
 
 /* myersVerifyDevice with the pipeline workspace in the device's static
