@@ -19,9 +19,14 @@ void verify_slice_kernel(myers_verify_args_t a, myers_queue_plan_t p, uint32_t m
     constexpr uint32_t kCands = (uint32_t)SliceShape<SL>::kCands;
     constexpr uint32_t kHead = MYERS_QUEUE_HEAD(SL == 16 ? MYERS_QUEUE_ONE_LANE_16 : MYERS_QUEUE_ONE_LANE);
     uint32_t next = blockIdx.x, lo = 0, hi = 0, part = 0;
-    // Workgroups are dispatched round-robin over the 8 XCDs; renumber them so
-    // that each XCD (own L2) takes a contiguous run of chunks.
-    if ((gridDim.x & 7u) == 0u) next = (blockIdx.x & 7u) * (gridDim.x >> 3) + (blockIdx.x >> 3);
+    if (mode == (uint32_t)MYERS_SLICE_PLAIN && (gridDim.x & 7u) == 0u) {
+        // Workgroups are dispatched round-robin over the 8 XCDs; renumber them so
+        // that each XCD (own L2) takes a contiguous run of chunks.  Not where the
+        // bin has fewer chunks than the grid workgroups: the first XCDs would take
+        // them all (200K candidates of 36-400 bases, a launch per bin: 1.0 ms, 0.56).
+        const uint32_t n = a.bin_ranges != nullptr ? a.bin_ranges[2u * p.variant[0] + 1u] : a.count;
+        if (n > (gridDim.x - 1u) * kCands) next = (blockIdx.x & 7u) * (gridDim.x >> 3) + (blockIdx.x >> 3);
+    }
     for (;;) {
         uint32_t j = 0, start = a.start, count = a.count, chunk = 0;
         if (mode == (uint32_t)MYERS_SLICE_QUEUE) {

@@ -47,10 +47,14 @@ def log(msg):
 
 
 def candidates_for(variants, w):
+    """Variants timed for w words.  Of the one-lane ones only that of w words: the
+    persistent engine has a bin per word count of short reads whatever a row says,
+    so the others would take the same time, and the engines with a launch per bin
+    the more the wider the row."""
     out = []
     for i, v in enumerate(variants):
         t = v["lanes"] * v["words"]
-        if t >= w and t <= max(2 * w, w + 4):
+        if t >= w and t <= max(2 * w, w + 4) and (v["lanes"] > 1 or v["words"] == w):
             out.append(i)
     return out
 
