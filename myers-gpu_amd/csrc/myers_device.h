@@ -75,12 +75,10 @@ __device__ __forceinline__ uint32_t sanitize_text(uint32_t w) {
     return c & ~((hi & lo) * 7u);
 }
 
-// Under-threshold bound k = (uint32)((float)m * e) (src/checksum-2.c:88), kept
-// small enough that the kernels' sums with it stay within 31 bits: no score is
-// above its read's length, so a larger bound lets the same candidates through.
-constexpr uint32_t kMaxThreshold = 1u << 24;
+// Under-threshold bound k = (uint32)((float)m * e) (src/checksum-2.c:88); the host
+// passes no e above MYERS_MAX_THRESHOLD, so that sums with k stay within 31 bits.
 __device__ __forceinline__ uint32_t threshold_of(uint32_t m, float e) {
-    return min((uint32_t)__fmul_rn((float)m, e), kMaxThreshold);
+    return (uint32_t)__fmul_rn((float)m, e);
 }
 
 __device__ __forceinline__ uint32_t wave_max(uint32_t v) {

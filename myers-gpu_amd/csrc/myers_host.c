@@ -1585,6 +1585,12 @@ static uint64_t nominal_cells(const qryInfo_t *qinfo, const candInfo_t *cands, u
     return cells;
 }
 
+/* The threshold as the kernels take it (< 0: off). */
+static float kernel_threshold(const myers_buffer_t *b)
+{
+    return b->threshold < MYERS_MAX_THRESHOLD ? b->threshold : MYERS_MAX_THRESHOLD;
+}
+
 /* Whether a batch's one launch reads and writes the pinned host arrays itself:
  * one-lane reads of one bin in a batch that is not binned (every array is then
  * read about once, and the launch does not wait for three copies, nor the caller
@@ -1647,7 +1653,7 @@ int myersSendEx(void *myersBuffer, float distance, uint32_t numPEQEntries, uint3
         SEND_TRY(hipMemcpyAsync(b->d_cands, b->h_cands, (size_t)numCandidates * sizeof(candInfo_t), hipMemcpyHostToDevice, s));
     const batch_t bt = {direct ? b->hd_peq : (void *)b->d_peq, direct ? b->hd_qinfo : (void *)b->d_qinfo,
                         direct ? b->hd_cands : (void *)b->d_cands, direct ? b->hd_results : (void *)b->d_results,
-                        numPEQEntries, numQueries, numCandidates, flags, distance, b->threshold, b->d_work, b->d_order,
+                        numPEQEntries, numQueries, numCandidates, flags, distance, kernel_threshold(b), b->d_work, b->d_order,
                         spare_list(b, numPEQEntries, numCandidates), b};
     rc = enqueue_verify(b, &bt, b->h_qinfo, b->h_cands);
     if (rc) return (b->last_error = rc);
@@ -1700,7 +1706,7 @@ int myers_serve_plan(void *myersBuffer, myers_serve_plan_t *out)
     out->d_ref = ctx->d_ref;
     out->ref_words = ctx->ref_words_alloc;
     out->ref_size = ctx->ref_size;
-    out->threshold = b->threshold;
+    out->threshold = kernel_threshold(b);
     uint32_t var_of[MYERS_SERVE_MAX_WORDS + 1];
     uint64_t used = 0;
     const uint32_t maxw = max_supported_words(ctx);
@@ -1781,7 +1787,7 @@ static int verify_device(myers_buffer_t *b, const void *d_peq, uint32_t numPEQEn
     if (rc) return (b->last_error = rc);
     *b->h_err = 0;
     const batch_t bt = {d_peq, d_qinfo, d_candidates, d_results, numPEQEntries, numQueries, numCandidates,
-                        flags, distance, b->threshold, d_work, d_order, d_list, pool_of};
+                        flags, distance, kernel_threshold(b), d_work, d_order, d_list, pool_of};
     rc = enqueue_verify(b, &bt, h_qinfo, NULL);
     b->stats.cells = 0;
     b->stats.candidates = numCandidates;

@@ -30,6 +30,9 @@ typedef struct {
     uint32_t block;          /* threads per workgroup: 64, or L for L > 64 (L/64 waves) */
 } myers_variant_desc_t;
 
+/* Highest threshold that the kernels take: no score is above its read's length, so
+ * higher ones let the same candidates through. */
+#define MYERS_MAX_THRESHOLD 2.0f
 typedef struct {
     const uint32_t *ref;         /* packed reference + guard words (all-N) */
     uint64_t        ref_words;   /* words readable at ref (incl. guard) */
