@@ -594,18 +594,22 @@ __device__ __noinline__ bool slice_run(SliceBatch a, SliceLds *lds_at) {
 // every one up to kFallbackExact words, where it also runs bins of its own
 // (small batches), above it those of the tuning table's bins, where a bin of
 // several word counts gives many chunks that the sliced form does not take (200-1000
-// bases, a launch per bin: 4.0 ms with 12, 16, 24 and 32, 3.7 ms).
+// bases, a launch per bin: 4.0 ms with 12, 16, 24 and 32, 3.7 ms).  Those that a
+// form has no reads for are left out of its kernel.
 constexpr uint32_t kFallbackExact = 7;
 #define SLICE_FALLBACK_WIDTHS(X)                                                                 \
     X(1) X(2) X(3) X(4) X(5) X(6) X(7) X(9) X(10) X(13) X(16) X(19) X(22) X(25) X(29) X(32)
+template <int SL>
 __device__ __forceinline__ void slice_fallback(const myers_verify_args_t &a, uint32_t start, uint32_t count,
-                                               uint32_t chunk, uint32_t lanes, uint32_t words, uint4 *lds) {
-    const uint32_t sub = 32u / lanes;
-    const uint32_t lo = chunk * sub, hi = min(lo + sub, (count + 63u) / 64u);
+                                               uint32_t chunk, uint32_t words, uint4 *lds) {
+    constexpr uint32_t kSub = 32u / (uint32_t)SL;
+    const uint32_t lo = chunk * kSub, hi = min(lo + kSub, (count + 63u) / 64u);
 #define SLICE_FALLBACK(WF)                                                                       \
-    if (words <= (WF)) {                                                                         \
-        verify_chunks<1, (WF), false>(a, start, count, lo, hi, 1u, *reinterpret_cast<Workspace<1, (WF)> *>(lds)); \
-        return;                                                                                  \
+    if constexpr ((WF) <= slice_max_words(SL) + 1) {                                             \
+        if (words <= (WF)) {                                                                     \
+            verify_chunks<1, (WF), false>(a, start, count, lo, hi, 1u, *reinterpret_cast<Workspace<1, (WF)> *>(lds)); \
+            return;                                                                              \
+        }                                                                                        \
     }
     SLICE_FALLBACK_WIDTHS(SLICE_FALLBACK)
 #undef SLICE_FALLBACK

@@ -89,7 +89,7 @@ void verify_slice_kernel(myers_verify_args_t a, myers_queue_plan_t p, uint32_t m
             if (done == kSliceShort) done = verify_slice<SL>(a, start, count, chunk, words, 0u, p.variant[j], slice_lds);
         }
         if (done != kSliceDone)
-            slice_fallback(a, start, count, chunk, (uint32_t)SL, words, slice_lds);
+            slice_fallback<SL>(a, start, count, chunk, words, slice_lds);
     }
 }
 
