@@ -128,10 +128,12 @@ int myersReceiveEx(void *myersBuffer);
  * minimum score is <= (uint32)((float)m * errorRate) exactly as without the
  * threshold, and every other verified candidate as
  * {column 0xFFFFFFFF, score 0xFFFFFFFF}; skipped candidates keep
- * {0, 0xFFFFFFFF}.  Large batches of queries of 545 to 1024 bases then run
+ * {0, 0xFFFFFFFF}.  Batches of many queries of 545 to 1024 bases then run
  * the first rows of every candidate and all rows of those only that these do
- * not rule out, and the multi-lane kernels of queue and per-bin launches stop
- * a wave once none of its candidates can get under the threshold.
+ * not rule out, smaller ones of one length skip the rows whose distance already
+ * exceeds a low threshold (Ukkonen cut-off), and the multi-lane kernels of queue
+ * and per-bin launches stop a wave once none of its candidates can get under the
+ * threshold.
  * errorRate < 0 switches the mode off (the default). */
 #define MYERS_NO_MATCH 0xFFFFFFFFu
 int   myersSetThreshold(void *myersBuffer, float errorRate);

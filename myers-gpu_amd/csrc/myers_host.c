@@ -726,17 +726,50 @@ static int large_batch(const myers_ctx_t *ctx, uint32_t num_cands)
     return (uint64_t)num_cands >= (uint64_t)ctx->num_cus * 2048u;
 }
 
+/* Threshold mode: whether the one-lane launch runs the first rows of its candidates
+ * first (slice_first_rows) and the rest of those kept in a second launch.
+ *
+ * The rows left out save their share of the bins' time, which batches of a round
+ * or two of waves spend at about 125e12 cells per second; the second launch takes
+ * one chunk of its kernel and 0.25 ms of launches, binning and tail.  8 candidates
+ * per read, threshold 0.05 m, all rows and first rows: 100K candidates of 1000 bases
+ * 1.04 and 1.15 ms, 150K 1.33 and 1.17; 100K of 800 0.69 and 0.84, 200K 1.15 and
+ * 0.92; 150K of 600 0.55 and 0.60, 400K 1.13 and 0.89; 250K of six lengths from 100
+ * to 1000 1.08 and 1.12. */
+#define FIRST_ROWS_MIN_CANDS 384u        /* per CU: below, all rows whatever the reads */
+static int first_rows_pay(const myers_ctx_t *ctx, const bin_scan_t *scan, const batch_t *bt)
+{
+    if (bt->threshold < 0.0f || bt->d_list == NULL || bt->num_queries == 0 ||
+        (uint64_t)bt->num_cands < (uint64_t)FIRST_ROWS_MIN_CANDS * (uint64_t)ctx->num_cus)
+        return 0;
+    if (!scan->sized) return (uint64_t)bt->num_cands >= 1024u * (uint64_t)ctx->num_cus;
+    const double cpr = (double)bt->num_cands / (double)bt->num_queries;
+    double saved = 0.0, second = 0.0;                /* ns */
+    for (uint64_t left = scan->present & ~ctx->multi_lane; left; left &= left - 1u) {
+        const uint32_t v = (uint32_t)__builtin_ctzll(left);
+        const double m = 32.0 * (double)ctx->variants[v].words;
+        const double share = myers_slice_first_rows(ctx->variants[v].words, bt->threshold) * 32.0 / m;
+        if (share <= 0.0) continue;
+        const double cands = scan->counted ? (double)scan->cands[v] : (double)scan->reads[v] * cpr;
+        const double chunk = (1.25 * m + 96.0) * (60.0 + 28.0 * (double)((ctx->variants[v].words + 1u) / 2u));
+        saved += (1.0 - share) * cands * 1.2 * m * m / 125e3;
+        if (chunk > second) second = chunk;
+    }
+    return saved > second + 250e3;
+}
+
 /* Auto: mixed lengths go to the persistent engine.  A batch of one length bin
  * runs on the plain engine (no binning pass) unless it holds more than ~2.7
  * rounds of what the chip keeps resident (2048 candidates per CU): there the
  * queue launch's pulls leave a shorter tail than one workgroup per chunk
- * (1.1M candidates of 1,000 bases: 8.70 against 8.78 ms). */
-static uint32_t resolve_engine(const myers_ctx_t *ctx, uint32_t flags, const bin_scan_t *scan, uint32_t num_cands)
+ * (1.1M candidates of 1,000 bases: 8.70 against 8.78 ms), or threshold mode's first
+ * rows pay, which need the binning's ranges. */
+static uint32_t resolve_engine(const myers_ctx_t *ctx, const bin_scan_t *scan, const batch_t *bt, int first_rows)
 {
-    uint32_t engine = flags & MYERS_ENGINE_MASK;
+    uint32_t engine = bt->flags & MYERS_ENGINE_MASK;
     if (engine == MYERS_ENGINE_AUTO) {
         const int single = scan->num_present == 1 && !scan->too_long;
-        engine = (single && !large_batch(ctx, num_cands)) ? MYERS_ENGINE_PLAIN : MYERS_ENGINE_PERSISTENT;
+        engine = (single && !large_batch(ctx, bt->num_cands) && !first_rows) ? MYERS_ENGINE_PLAIN : MYERS_ENGINE_PERSISTENT;
     }
     return engine;
 }
@@ -1153,17 +1186,42 @@ static uint32_t split_plan(const myers_ctx_t *ctx, const bin_scan_t *scan, const
     return words;
 }
 
+/* The cut-off kernel for a bin of reads of up to `words` words with about `cands`
+ * candidates in threshold mode (its variant), or -1: the sliced kernel.
+ *
+ * Low thresholds leave the cut-off a few rows per column: 8 candidates per read of
+ * 1000 bases, threshold 0.05 m, 20K candidates 0.73 ms against 0.81 with the sliced
+ * kernel, 100K 0.95 against 1.04; 0.1 m 0.77 and 0.81, 0.98 and 1.02; 0.2 m 0.83 and
+ * 0.81.  Shorter reads' sliced chunks take less time than the cut-off's unless
+ * waves share the SIMDs (800 bases, 0.05 m: 50K 0.49 and 0.47, 100K 0.63 and 0.69;
+ * 600 bases 0.31 and 0.30, 0.40 and 0.42); at 400 bases it gains nothing. */
+static int cut_variant(const myers_ctx_t *ctx, uint32_t words, float threshold, double cands)
+{
+    if (threshold < 0.0f || threshold > 0.1f || words < 17u ||
+        (words <= 28u && cands < 288.0 * (double)ctx->num_cus))
+        return -1;
+    for (uint32_t v = 0; v < ctx->num_variants; v++)
+        if (ctx->variants[v].lanes == 1u && ctx->variants[v].words >= words && myers_variant_cut_ok(v)) return (int)v;
+    return -1;
+}
+
 /* Launch one bin: variant v over a->start / count or its bin range, with a
  * fixed grid (resident = 0) or a resident grid that pulls from the variant's
  * part heads. */
-static int launch_bin(myers_ctx_t *ctx, uint32_t v, myers_verify_args_t *a, const slice_load_t *load, int resident,
-                      hipStream_t stream)
+static int launch_bin(myers_buffer_t *b, uint32_t v, myers_verify_args_t *a, const slice_load_t *load, double cands_in_bin,
+                      int resident, hipStream_t stream)
 {
+    myers_ctx_t *ctx = b->ctx;
+    b->ran.ran |= MYERS_RAN_BIN;
     const myers_variant_desc_t *d = &ctx->variants[v];
     const uint32_t num_cands = load->num_cands;
     a->variant = v;
     a->chunk_factor = ctx->chunk_factor[v];
     if (d->lanes == 1u) {
+        const int cut = resident ? -1 : cut_variant(ctx, d->words, a->threshold, cands_in_bin);
+        if (cut >= 0) b->ran.ran |= MYERS_RAN_CUT;
+        if (cut >= 0)
+            return myers_launch_verify((uint32_t)cut, a, grid_for(ctx, v, num_cands, a->bin_ranges != NULL), 0, stream);
         myers_queue_plan_t p;
         memset(&p, 0, sizeof(p));
         const uint32_t lanes = slice_lanes(ctx, d->words, load), cands = lanes == 16u ? 128u : 64u;
@@ -1264,8 +1322,9 @@ static int enqueue_pipeline(myers_buffer_t *b, const batch_t *bt, const bin_scan
     myers_split_plan_t sp;
     uint32_t split_grid = 0;
     const uint32_t split = wide ? 0u : split_plan(ctx, scan, bt, order, n, &sp, &split_grid);
+    const int first_rows = first_rows_pay(ctx, scan, bt);
     const uint32_t engine =
-        wide || split ? (uint32_t)MYERS_ENGINE_PERSISTENT : resolve_engine(ctx, bt->flags, scan, bt->num_cands);
+        wide || split ? (uint32_t)MYERS_ENGINE_PERSISTENT : resolve_engine(ctx, scan, bt, first_rows);
     b->stats.launches = 0;
     b->stats.variantsUsed = 0;
     b->binned = 0;
@@ -1282,9 +1341,9 @@ static int enqueue_pipeline(myers_buffer_t *b, const batch_t *bt, const bin_scan
         a.count = bt->num_cands;
         const uint32_t waves = (bt->num_cands + 3u) / 4u;
         rc = one_part ? myers_launch_split(&a, &sp, split, split_grid < waves ? split_grid : waves, b->stream)
-                      : launch_bin(ctx, v, &a, &load, 0, b->stream);
+                      : launch_bin(b, v, &a, &load, (double)bt->num_cands, 0, b->stream);
         if (rc) return hip_fail((hipError_t)rc, "verify launch", __FILE__, __LINE__);
-        b->ran.ran = one_part ? MYERS_RAN_SPLIT : MYERS_RAN_BIN;
+        if (one_part) b->ran.ran |= MYERS_RAN_SPLIT;
         b->ran.split_words = one_part ? split : 0u;
         b->stats.launches = 1;
         b->stats.variantsUsed = 1;
@@ -1334,9 +1393,12 @@ static int enqueue_pipeline(myers_buffer_t *b, const batch_t *bt, const bin_scan
     if (engine == MYERS_ENGINE_PLAIN) {
         /* one launch per length bin, in turn */
         for (uint32_t i = 0; i < n; i++) {
-            rc = launch_bin(ctx, order[i], &a, &load, 0, b->stream);
+            const uint32_t v = order[i];
+            const double cands = !scan->sized || bt->num_queries == 0 ? 0.0 :
+                                 scan->counted ? (double)scan->cands[v] :
+                                 (double)scan->reads[v] * (double)bt->num_cands / (double)bt->num_queries;
+            rc = launch_bin(b, v, &a, &load, cands, 0, b->stream);
             if (rc) return hip_fail((hipError_t)rc, "verify launch", __FILE__, __LINE__);
-            b->ran.ran |= MYERS_RAN_BIN;
         }
     } else {
         /* Persistent engines.  The long-read bins of a latency-bound batch
@@ -1370,10 +1432,6 @@ static int enqueue_pipeline(myers_buffer_t *b, const batch_t *bt, const bin_scan
             nother = nrest;
         }
         launches = (nlong ? 1u : 0u) + (split ? 1u : 0u) + nqueue + nother;
-        /* threshold mode, batches of more than a round of the one-lane kernel's
-         * waves (275K candidates of 1000 bases: 2.15 ms either way): the first
-         * rows first (slice_first_rows) */
-        const int can_filter = bt->threshold >= 0.0f && bt->d_list && (uint64_t)bt->num_cands >= 1024u * (uint64_t)ctx->num_cus;
         const int fork = launches > 1u;
         const uint32_t width = !fork ? 0u : (launches < SIDE_STREAMS ? launches : SIDE_STREAMS);
         uint32_t next = 0;    /* launches placed so far: launch k goes on side stream k % width */
@@ -1420,7 +1478,7 @@ static int enqueue_pipeline(myers_buffer_t *b, const batch_t *bt, const bin_scan
                 rc = myers_launch_queue(&a, &qp[c], grid, stream);
             } else {
                 myers_verify_args_t two = a;
-                const int filter = can_filter && c == (uint32_t)MYERS_QUEUE_ONE_LANE;
+                const int filter = first_rows && c == (uint32_t)MYERS_QUEUE_ONE_LANE;
                 if (filter) {
                     two.list = bt->d_list;
                     two.list_ranges = bt->d_work + MYERS_WORK_LIST;
@@ -1447,9 +1505,8 @@ static int enqueue_pipeline(myers_buffer_t *b, const batch_t *bt, const bin_scan
             if (rc) return hip_fail((hipError_t)rc, "queue launch", __FILE__, __LINE__);
         }
         for (uint32_t i = 0; i < nother; i++) {
-            rc = launch_bin(ctx, other[i], &a, &load, 1, NEXT_STREAM());
+            rc = launch_bin(b, other[i], &a, &load, 0.0, 1, NEXT_STREAM());
             if (rc) return hip_fail((hipError_t)rc, "persistent launch", __FILE__, __LINE__);
-            b->ran.ran |= MYERS_RAN_BIN;
         }
 #undef NEXT_STREAM
         for (uint32_t j = 0; j < width; j++) {
@@ -1539,7 +1596,8 @@ static int enqueue_verify(myers_buffer_t *b, const batch_t *bt, const qryInfo_t 
                               ((uint64_t)bt->num_cands << 32) | bt->flags,
                               (uint64_t)dist_bits, scan.present,
                               (uint64_t)scan.too_long, b->ctx->tune_gen, (uint64_t)thr_bits, plan_key,
-                              wide_bins(b->ctx, &scan, bt), (uint64_t)split | ((uint64_t)sp.n << 8) | ((uint64_t)split_grid << 32)};
+                              wide_bins(b->ctx, &scan, bt), (uint64_t)split | ((uint64_t)sp.n << 8) |
+                                  ((uint64_t)first_rows_pay(b->ctx, &scan, bt) << 31) | ((uint64_t)split_grid << 32)};
     if (!b->graph_valid || memcmp(key, b->graph_key, sizeof(key)) != 0) {
         if (b->graph_exec) {
             hipGraphExecDestroy(b->graph_exec);
@@ -1606,6 +1664,10 @@ static int reads_host_arrays(const myers_buffer_t *b, uint32_t flags, uint32_t n
         return 0;
     const uint32_t first = (b->h_qinfo[0].size + 31u) >> 5;
     if (first > 32u) return 0;
+    /* (such a batch may be binned: first_rows_pay) */
+    if (b->threshold >= 0.0f && (uint64_t)num_cands >= (uint64_t)FIRST_ROWS_MIN_CANDS * (uint64_t)b->ctx->num_cus &&
+        myers_slice_first_rows(first, b->threshold) != 0u)
+        return 0;
     const uint8_t *bin = bins_of(b->ctx, flags);
     for (uint32_t q = 1; q < num_queries; q++) {
         const uint32_t w = (b->h_qinfo[q].size + 31u) >> 5;

@@ -20,7 +20,8 @@ enum { MYERS_RAN_BIN = 1,            /* a launch per bin */
        MYERS_RAN_QUEUE = 16,         /* multi-lane queue launch */
        MYERS_RAN_LONG = 32,          /* long-read launch */
        MYERS_RAN_SPLIT = 64,         /* split launch */
-       MYERS_RAN_HANDOVERS = 128 };  /* ... of several parts per candidate */
+       MYERS_RAN_HANDOVERS = 128,    /* ... of several parts per candidate */
+       MYERS_RAN_CUT = 256 };        /* cut-off kernel of a bin's launch */
 typedef struct {
     uint32_t ran, split_words, split_slots;
 } myers_launch_info_t;

@@ -77,6 +77,9 @@ int      myers_variant_occupancy(uint32_t v, int *wg_per_cu);
  * is drained. */
 int myers_launch_verify(uint32_t v, const myers_verify_args_t *args, uint32_t grid,
                         int persistent, hipStream_t stream);
+/* 1 if one-lane variant v has a cut-off kernel, which myers_launch_verify then runs
+ * in threshold mode (plain launches). */
+int myers_variant_cut_ok(uint32_t v);
 /* Resident workgroups per CU of the persistent kernel of variant v. */
 int myers_variant_occupancy_persistent(uint32_t v, int *wg_per_cu);
 
@@ -167,6 +170,9 @@ int myers_launch_queue(const myers_verify_args_t *args, const myers_queue_plan_t
 enum { MYERS_SLICE_PLAIN = 0, MYERS_SLICE_RANGES = 1, MYERS_SLICE_QUEUE = 2 };
 uint32_t myers_slice_max_words(uint32_t lanes);
 uint32_t myers_slice_ws_u4(uint32_t lanes, uint32_t words);     /* LDS in 16-byte units, 0: no such form */
+/* Rows per lane that a queue launch with a list computes first for reads of `words`
+ * words (0: all rows at once). */
+uint32_t myers_slice_first_rows(uint32_t words, float threshold);
 int myers_slice_occupancy(uint32_t lanes, uint32_t lds_bytes, int *wg_per_cu);
 int myers_launch_slice(const myers_verify_args_t *args, const myers_queue_plan_t *plan, uint32_t mode, uint32_t grid,
                        hipStream_t stream);

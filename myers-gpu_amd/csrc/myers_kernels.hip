@@ -895,12 +895,17 @@ constexpr const void *cut_kernel(bool persistent) {
 }
 // One-lane variants run the kernels of myers_slice.hip; those of the shortest
 // reads have a plain bit-vector kernel for small batches of one length too
-// (110K candidates of 100 bases: 32 us, the sliced form 41).
+// (110K candidates of 100 bases: 32 us, the sliced form 41), and some wide ones
+// the cut-off kernel for low thresholds (launch_bin).
 constexpr int kPlainOneLane = 7;
+template <int W>
+constexpr bool kCutOneLane = W == 19 || W == 22 || W == 25 || W == 29 || W == 32;
 template <int L, int W>
 constexpr VariantEntry variant_entry() {
     if constexpr (L == 1 && W <= kPlainOneLane) {
         return {1u, (uint32_t)W, reinterpret_cast<const void *>(&verify_kernel<1, W, false>), nullptr, nullptr, nullptr, 64u};
+    } else if constexpr (L == 1 && kCutOneLane<W>) {
+        return {1u, (uint32_t)W, nullptr, nullptr, reinterpret_cast<const void *>(&verify_kernel<1, W, true>), nullptr, 64u};
     } else if constexpr (L == 1) {
         return {1u, (uint32_t)W, nullptr, nullptr, nullptr, nullptr, 64u};
     } else {
@@ -965,16 +970,19 @@ extern "C" int myers_variant_occupancy_persistent(uint32_t v, int *wg_per_cu) {
 
 extern "C" int myers_launch_verify(uint32_t v, const myers_verify_args_t *args, uint32_t grid,
                                    int persistent, hipStream_t stream) {
-    if (v >= kNumVariants || args == nullptr || grid == 0 || kVariants[v].fn == nullptr ||
-        (persistent && kVariants[v].persistent_fn == nullptr))
-        return -1;
+    if (v >= kNumVariants || args == nullptr || grid == 0) return -1;
     if (persistent && (args->bin_ranges == nullptr || args->queue_heads == nullptr)) return -1;
     void *kargs[] = {const_cast<myers_verify_args_t *>(args)};
     const VariantEntry &ve = kVariants[v];
     const bool cut = args->threshold >= 0.0f && ve.cut_fn != nullptr;
     const void *fn = cut ? (persistent ? ve.cut_persistent_fn : ve.cut_fn) : (persistent ? ve.persistent_fn : ve.fn);
+    if (fn == nullptr) return -1;
     hipError_t e = hipLaunchKernel(fn, dim3(grid), dim3(ve.block), kargs, 0, stream);
     return (int)e;
+}
+
+extern "C" int myers_variant_cut_ok(uint32_t v) {
+    return v < kNumVariants && kVariants[v].lanes == 1u && kVariants[v].cut_fn != nullptr;
 }
 
 extern "C" int myers_variant_long_ok(uint32_t v, uint32_t *ws_u4) {

@@ -626,11 +626,12 @@ __device__ __forceinline__ void slice_fallback(const myers_verify_args_t &a, uin
 // them at its place, k = 0.2 m: 50K reads of 1000 bases 3.83 -> 2.79 ms, 100K of
 // 600 bases 2.73 -> 2.43 ms; at 400 bases the work per column is most of a
 // chunk and the second launch takes what the first gains (1.56 -> 1.75 ms).
+// (k: the threshold of a read of max_words words)
 template <int SL>
-__device__ __forceinline__ uint32_t slice_first_rows(uint32_t max_words, float threshold) {
+__host__ __device__ __forceinline__ uint32_t slice_first_rows(uint32_t max_words, float k) {
     const float m = 32.0f * (float)max_words;
     const uint32_t all = 32u * max_words / (uint32_t)SL;
-    const float r = 2.05f * (float)threshold_of(32u * max_words, threshold) + 0.75f * sqrtf(m) + 6.0f;
+    const float r = 2.05f * k + 0.75f * sqrtf(m) + 6.0f;
     const uint32_t rows = r >= m ? all : ((uint32_t)r + (uint32_t)SL) / (uint32_t)SL;
     return SL == 32 && max_words >= 18u && 10u * rows <= 7u * all ? rows : 0u;
 }

@@ -77,7 +77,7 @@ void verify_slice_kernel(myers_verify_args_t a, myers_queue_plan_t p, uint32_t m
         if (p.key[j] >> 8 != 1u) {
             // first rows only, while they rule out enough: of `tally`'s
             // candidates a share below 0.75 of what the rows left out would cost
-            uint32_t first = a.list != nullptr ? slice_first_rows<SL>(words, a.threshold) : 0u;
+            uint32_t first = a.list != nullptr ? slice_first_rows<SL>(words, (float)threshold_of(32u * words, a.threshold)) : 0u;
             if (first != 0u) {
                 const uint32_t tried = __hip_atomic_load(a.tally, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
                 const uint32_t kept = __hip_atomic_load(a.tally + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -133,6 +133,10 @@ __global__ __launch_bounds__(256) void planes_kernel(const uint32_t *ref, uint64
 extern "C" uint32_t myers_slice_max_words(uint32_t lanes) {
     if (lanes == 1u) return kFallbackExact;
     return lanes == 16u || lanes == 32u ? (uint32_t)slice_max_words((int)lanes) : 0u;
+}
+
+extern "C" uint32_t myers_slice_first_rows(uint32_t words, float threshold) {
+    return slice_first_rows<32>(words, floorf(32.0f * (float)words * threshold));
 }
 
 extern "C" uint32_t myers_slice_ws_u4(uint32_t lanes, uint32_t words) {

@@ -3,7 +3,7 @@ import ctypes
 
 import myers_amd as M
 
-BIN, SLICE, FIRST_ROWS, WIDE_SLICE, QUEUE, LONG, SPLIT, HANDOVERS = (1 << k for k in range(8))
+BIN, SLICE, FIRST_ROWS, WIDE_SLICE, QUEUE, LONG, SPLIT, HANDOVERS, CUT = (1 << k for k in range(9))
 
 
 class Info(ctypes.Structure):

@@ -32,21 +32,21 @@ def test_creation():
     assert per_buffer < (2 + 1.1 + 6 * 2) * MIB, per_buffer / MIB
 
 
-@pytest.mark.parametrize("fill,entries,first_rows", [(1.0, 0, False), (0.9, 0, False), (0.9, 60_000, True),
+@pytest.mark.parametrize("fill,entries,first_rows", [(1.0, 0, False), (0.9, 0, False), (0.9, 40_000, True),
                                                      (0.75, 0, True)])
 def test_list_of_the_second_launch(fill, entries, first_rows):
     """Threshold mode over a batch that fills the buffer: the first rows run where
     the candidates or the Peq entries leave room for the list."""
     ref = M.synth_reference(96, SIZE)
     reads = 66_000
-    b = M.synth_batch(M.make_spec(7, reads, choices=[600, 300], err_range=(0.0, 0.2), candidates=5, distance=0.1), ref,
+    b = M.synth_batch(M.make_spec(7, reads, choices=[1000, 900], err_range=(0.0, 0.2), candidates=5, distance=0.1), ref,
                       SIZE)
     nc, ne = len(b["cands"]), len(b["peq"])
     full = O.myers_batch(ref, SIZE, b["peq"], b["qinfo"], b["cands"], 0.1, M.WINDOW_ALIGNED)
     want = O.apply_threshold(b["qinfo"], b["cands"], full, 0.1)
     # the capacities: avg_query's entries per read, and bytes for nc / fill candidates
-    per_cand = (5 * 80 + 8) / 5 + 28
-    with M.Myers(ref, SIZE, avg_query=640, cands_per_query=5, buffer_bytes=int(nc / fill * per_cand) + 200) as m:
+    per_cand = (8 * 80 + 8) / 5 + 28
+    with M.Myers(ref, SIZE, avg_query=1000, cands_per_query=5, buffer_bytes=int(nc / fill * per_cand) + 200) as m:
         cap_e, _, cap_c = m.capacity()
         peq = np.zeros((cap_e - entries, 20), np.uint32)            # spare entries at the end
         peq[:ne] = b["peq"]
