@@ -72,6 +72,7 @@ typedef struct myers_ctx {
     uint8_t   bin_of_words[BIN_ROWS];              /* the caller's table or the tuning file's */
     uint8_t   fine_of_words[BIN_ROWS];             /* the same with a bin per word count of one-lane reads (bins_of) */
     uint8_t  *d_bin_of_words;                      /* both, one after the other */
+    uint32_t  in_flight;         /* buffers with a batch sent and not yet received */
     uint64_t  tune_gen;          /* bumped when the bin table or chunk factors change */
     uint32_t *d_scratch;         /* this device's static workspace (myersVerifyDeviceNoAlloc) */
 } myers_ctx_t;
@@ -719,6 +720,7 @@ typedef struct {
     uint32_t   *d_order;     /* slot -> candidate, num_cands words */
     uint32_t   *d_list;      /* num_cands words, or NULL */
     myers_buffer_t *pool_of; /* the buffer whose pool the split launch may use, or NULL */
+    double      share;       /* of the chip that the batch can expect (chip_share) */
 } batch_t;
 
 static int large_batch(const myers_ctx_t *ctx, uint32_t num_cands)
@@ -861,7 +863,7 @@ static uint32_t long_plan(const myers_ctx_t *ctx, const bin_scan_t *scan, const 
         work = work_wide;
     }
     if (ns) {
-        *ns = work / simds;
+        *ns = work / (simds * bt->share);
         for (uint32_t k = 0; k < nt; k++)
             if (chain[k] > *ns) *ns = chain[k];
     }
@@ -1101,7 +1103,10 @@ static uint32_t *split_pool(myers_buffer_t *b)
  * where that is one bin of one part per candidate without binning (8 candidates
  * per read: 100 reads of 100 bases 31 us against 34 with the bit-vector kernel,
  * 200 reads would be 35.5 against 34.5; 100 reads of 250 bases 41 against 88, of
- * 1000 bases 87 against 680, 1,000 reads of 1000 bases 415 against 680). */
+ * 1000 bases 87 against 680, 1,000 reads of 1000 bases 415 against 680).
+ * The split launch spends more of the chip per cell than the launches it stands
+ * in for (60-98e12 cells per second against 110-130e12), so a batch beside others
+ * weighs the work with its share of the chip. */
 static uint32_t split_plan(const myers_ctx_t *ctx, const bin_scan_t *scan, const batch_t *bt, const uint32_t *order,
                            uint32_t n, myers_split_plan_t *sp, uint32_t *grid)
 {
@@ -1113,7 +1118,7 @@ static uint32_t split_plan(const myers_ctx_t *ctx, const bin_scan_t *scan, const
         (engine != MYERS_ENGINE_AUTO && engine != MYERS_ENGINE_PERSISTENT))
         return 0;
     const double cpr = (double)bt->num_cands / (double)bt->num_queries;
-    const double simds = 4.0 * (double)ctx->num_cus;
+    const double simds = 4.0 * (double)ctx->num_cus * bt->share, rate = 120e3 * bt->share;
     /* the binning, which a batch of one bin does without, also here if it is one
      * part per candidate */
     const int one = engine == MYERS_ENGINE_AUTO && scan->num_present == 1;
@@ -1138,7 +1143,7 @@ static uint32_t split_plan(const myers_ctx_t *ctx, const bin_scan_t *scan, const
         myers_long_plan_t lp;
         /* (a quarter of a chain: what the tail of the long-read launch took over its estimate) */
         if (scan->num_present > 1 && long_plan(ctx, scan, bt, order, n, &lp, &old)) old += 0.25 * old_chain;
-        else old = cells / 120e3 > old_chain ? cells / 120e3 : old_chain;
+        else old = cells / rate > old_chain ? cells / rate : old_chain;
         now = split_est_ns(&est, simds, &best);
         if (one && ctx->variants[sp->variant[0]].total_words > 64u * split_kinds[best].words) extra = 50e3;
         if (now + extra >= old) return 0;
@@ -1153,7 +1158,7 @@ static uint32_t split_plan(const myers_ctx_t *ctx, const bin_scan_t *scan, const
         const double m = (double)scan->max_m[v];
         double chunk = d->words < 8u ? 1.25 * m * (40.0 + 20.0 * (double)d->words)
                                      : (1.25 * m + 31.0) * (20.0 + 16.6 * (double)d->words);
-        if (cands * 1.25 * m * m / 220e3 > chunk) chunk = cands * 1.25 * m * m / 220e3;
+        if (cands * 1.25 * m * m / (220e3 * bt->share) > chunk) chunk = cands * 1.25 * m * m / (220e3 * bt->share);
         if (chunk > slowest) slowest = chunk;
         split_est_t with = est;
         uint32_t kind = 0;
@@ -1643,6 +1648,26 @@ static uint64_t nominal_cells(const qryInfo_t *qinfo, const candInfo_t *cands, u
     return cells;
 }
 
+/* The share of the chip that a batch of this buffer can expect beside the library's
+ * other buffers with a batch in flight.  One other is mostly near its end when the
+ * batch starts; two count for half of it (three buffers served at 16.5e6 candidates
+ * per second of the serving mix: p50 11.5 ms and p99 27 ms as if alone, 10.1 and 21.5;
+ * at 8e6 4.2 ms either way, 5.3 if every other counted for one).  A captured pipeline
+ * runs beside whatever its replays meet, and keeps one plan. */
+static double chip_share(const myers_buffer_t *b, uint32_t flags)
+{
+    if (flags & MYERS_USE_GRAPH) return 1.0;
+    const uint32_t others = __atomic_load_n(&b->ctx->in_flight, __ATOMIC_RELAXED) - (b->pending ? 1u : 0u);
+    return others > 1u ? 2.0 / (1.0 + (double)others) : 1.0;
+}
+
+static void set_pending(myers_buffer_t *b, int pending)
+{
+    if (pending && !b->pending) __atomic_fetch_add(&b->ctx->in_flight, 1u, __ATOMIC_RELAXED);
+    if (!pending && b->pending) __atomic_fetch_sub(&b->ctx->in_flight, 1u, __ATOMIC_RELAXED);
+    b->pending = pending;
+}
+
 /* The threshold as the kernels take it (< 0: off). */
 static float kernel_threshold(const myers_buffer_t *b)
 {
@@ -1716,7 +1741,7 @@ int myersSendEx(void *myersBuffer, float distance, uint32_t numPEQEntries, uint3
     const batch_t bt = {direct ? b->hd_peq : (void *)b->d_peq, direct ? b->hd_qinfo : (void *)b->d_qinfo,
                         direct ? b->hd_cands : (void *)b->d_cands, direct ? b->hd_results : (void *)b->d_results,
                         numPEQEntries, numQueries, numCandidates, flags, distance, kernel_threshold(b), b->d_work, b->d_order,
-                        spare_list(b, numPEQEntries, numCandidates), b};
+                        spare_list(b, numPEQEntries, numCandidates), b, chip_share(b, flags)};
     rc = enqueue_verify(b, &bt, b->h_qinfo, b->h_cands);
     if (rc) return (b->last_error = rc);
     if (numCandidates && !direct)
@@ -1725,7 +1750,7 @@ int myersSendEx(void *myersBuffer, float distance, uint32_t numPEQEntries, uint3
 #undef SEND_TRY
     b->stats.cells = nominal_cells(b->h_qinfo, b->h_cands, numCandidates, distance);
     b->stats.candidates = numCandidates;
-    b->pending = 1;
+    set_pending(b, 1);
     b->last_error = MYERS_SUCCESS;
     return MYERS_SUCCESS;
 }
@@ -1739,7 +1764,7 @@ static int finish_batch(myers_buffer_t *b, int with_batch_events)
         if (rc) return rc;
     }
     if (!b->pending) return MYERS_SUCCESS;
-    b->pending = 0;
+    set_pending(b, 0);
     float ms = 0.0f;
     if (with_batch_events && hipEventElapsedTime(&ms, b->ev_batch_start, b->ev_batch_end) == hipSuccess)
         b->stats.batchMs = ms;
@@ -1849,11 +1874,11 @@ static int verify_device(myers_buffer_t *b, const void *d_peq, uint32_t numPEQEn
     if (rc) return (b->last_error = rc);
     *b->h_err = 0;
     const batch_t bt = {d_peq, d_qinfo, d_candidates, d_results, numPEQEntries, numQueries, numCandidates,
-                        flags, distance, kernel_threshold(b), d_work, d_order, d_list, pool_of};
+                        flags, distance, kernel_threshold(b), d_work, d_order, d_list, pool_of, chip_share(b, flags)};
     rc = enqueue_verify(b, &bt, h_qinfo, NULL);
     b->stats.cells = 0;
     b->stats.candidates = numCandidates;
-    b->pending = (rc == MYERS_SUCCESS);
+    set_pending(b, rc == MYERS_SUCCESS);
     b->last_error = rc;
     return rc;
 }
