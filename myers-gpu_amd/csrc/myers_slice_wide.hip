@@ -502,7 +502,11 @@ extern "C" int myers_launch_wide_slice(const myers_verify_args_t *args, const my
         const uint32_t team = myers_wide_slice_team(d.total_words);
         if (team == 0u || plan->key[j] != team) return -1;
     }
+    const size_t lds = (size_t)WideSlice::ws_u4() * 16u;
+    const void *fn = reinterpret_cast<const void *>(&verify_wide_slice_kernel);
+    // above 64 KiB a launch needs the kernel's limit raised (as myers_launch_long)
+    const hipError_t e = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+    if (e != hipSuccess) return (int)e;
     void *kargs[] = {const_cast<myers_verify_args_t *>(args), const_cast<myers_queue_plan_t *>(plan)};
-    return (int)hipLaunchKernel(reinterpret_cast<const void *>(&verify_wide_slice_kernel), dim3(grid),
-                                dim3(64u * WideSlice::kWaves), kargs, (size_t)WideSlice::ws_u4() * 16u, stream);
+    return (int)hipLaunchKernel(fn, dim3(grid), dim3(64u * WideSlice::kWaves), kargs, lds, stream);
 }
