@@ -77,11 +77,10 @@ CONFIGS = {
         log_uniform=(2000, 20000), err_range=(0.12, 0.12), sub_frac=0.5, candidates=4)),
 }
 DISTANCE = 0.1
-# HBM bytes per launch of the dominant kernel under the auto engine (the queue
-# launch for each), from FETCH_SIZE and WRITE_SIZE counter runs scaled by a 1 GiB
-# copy calibration (profiles/verify_queue_kernel_config2.md,
-# profiles/hbm_traffic_verify_queue_config3.md, profiles/hbm_traffic_verify_queue_config4.md).
-MEASURED_TRAFFIC = {(2, "aligned"): 1.624e9, (3, "aligned"): 9.547e9, (4, "aligned"): 1.536e9}
+# HBM bytes of a step's verification launches under the auto engine (the sliced
+# kernels), from FETCH_SIZE and WRITE_SIZE counter runs scaled by a 1 GiB copy
+# calibration (profiles/hbm_traffic_sliced_kernels.md).
+MEASURED_TRAFFIC = {(2, "aligned"): 2.269e9, (3, "aligned"): 16.45e9, (4, "aligned"): 2.153e9}
 
 
 def log(msg):
@@ -425,7 +424,7 @@ def roofline(cells, kernel_ms, hbm_bytes, traffic, kernel):
         "unit": "TOP/s",
         "frac": achieved / PEAK_VALU_OPS,
         "traffic": traffic,
-        "traffic_unit": "bytes/launch (rocprofv3 FETCH_SIZE + WRITE_SIZE, copy-calibrated)",
+        "traffic_unit": "bytes/step's verification launches (rocprofv3 FETCH_SIZE + WRITE_SIZE, copy-calibrated)",
         "kernel": kernel,
         "kernel_ms": kernel_ms,
         "ops_per_cell": K_GFX950 / 32.0,
@@ -448,12 +447,14 @@ def variant_names(m, b):
 
 def dominant_kernel(m, b, engine, run):
     """Name of the launch the roofline is taken over."""
-    names = variant_names(m, b)
-    if not run["binned"]:
-        return f"verify_kernel<{names[0][1:].replace('xW', ', ')}, false> (one launch)"
-    if engine in (M.ENGINE_PERSISTENT, M.ENGINE_AUTO) and run["launches"] == 1:
-        return "verify_queue_kernel (one launch over every bin: " + ", ".join(names) + ")"
-    return f"{run['launches']:.0f} launches ({', '.join(names)})"
+    names = ", ".join(variant_names(m, b))
+    longest = int(b["qinfo"][:, 1].max())
+    if run["launches"] == 1:
+        kernel = "verify_slice_kernel" if longest <= 1024 else "verify_wide_slice_kernel"
+        if engine not in (M.ENGINE_PERSISTENT, M.ENGINE_AUTO):
+            kernel = "one bin's kernel"
+        return f"{kernel} (one launch: {names})"
+    return f"{run['launches']:.0f} launches ({names})"
 
 
 def measure_config(m, ref, cfg_id, steps, warmup, engine, mode, graph, compare, cpu_seconds, threshold=-1.0):

@@ -66,9 +66,10 @@ typedef struct myers_ctx {
     uint64_t  multi_lane, deep;   /* masks: variants of several lanes; one-lane ones of 8 words or more */
     uint32_t  chunk_factor[MYERS_MAX_VARIANTS];    /* persistent: chunks per queue pull */
     uint32_t  long_seq;                            /* long-read launches so far (placement rotation) */
-    int       queue_occ[4];                        /* workgroups per CU of the multi-lane queue kernel, its
-                                                      threshold form and the two one-lane kernels, */
-    uint32_t  queue_occ_lds[4];                    /* for this dynamic LDS size (0: not queried) */
+    /* workgroups per CU of the multi-lane queue kernel, its threshold form and the two
+     * one-lane kernels, each for the dynamic LDS size beside it (0: not queried) */
+    int       queue_occ[4];
+    uint32_t  queue_occ_lds[4];
     uint8_t   bin_of_words[BIN_ROWS];              /* the caller's table or the tuning file's */
     uint8_t   fine_of_words[BIN_ROWS];             /* the same with a bin per word count of one-lane reads (bins_of) */
     uint8_t  *d_bin_of_words;                      /* both, one after the other */
